@@ -87,14 +87,12 @@ ENGINE_TUNE = {}
 
 # profiled kernel classes of the elastic time step (fwi3d_profile_read), by step form
 KERNEL_CLASSES = {
-    True: ((0, "elastic_fused"), (1, "elastic_flux_yfaces"), (3, "elastic_yslabs")),
+    True: ((0, "elastic_fused"),),
     False: ((0, "elastic_interior"), (1, "elastic_flux"), (2, "elastic_boundary"), (3, "elastic_zslab")),
 }
 STEP_KERNEL = {
-    True: "elastic time step = elastic_fused_batch (middle and edge tiles, planes [6, ny-6)) + elastic_flux_batch "
-          "(the 8 planes at each y face) + elastic_yslabs_ext (y-face slabs, edges, receivers) launches, the edge "
-          "tiles on a second stream beside the middle tiles and the y-face launches after the middle tiles (HIP "
-          "events around each step on the engine stream; the per-kernel averages come from a run with one stream)",
+    True: "elastic time step = one elastic_fused_step launch (all tiles and the receivers; HIP events around each "
+          "step on the engine stream)",
     False: "elastic time step = elastic_flux + elastic_interior + elastic_boundary + elastic_zslab launches "
            "(HIP events around each step on the engine stream)",
 }
@@ -116,16 +114,12 @@ def traffic_profile(n):
 
 def kernel_rooflines(fused, nz, nx, ny, avg_us, n):
     """Per kernel class of the elastic step: the cells it handles, its algorithmic bytes
-    (48 B per cell it updates: u, prev, lambda, mu, rho read, next written; the y-face
-    flux pass reads u, lambda, mu and writes T and 6 fluxes, 48 B per cell too), its
-    one-stream launch time, achieved GB/s and fraction of 8 TB/s, and its measured HBM
+    (48 B per cell it updates: u, prev, lambda, mu, rho read, next written), its launch time, achieved GB/s and fraction of 8 TB/s, and its measured HBM
     bytes per launch from the committed PMC summary when there is one."""
     nxz = nx * nz
     if fused:
-        cells = {"elastic_fused": nxz * max(0, ny - 12), "elastic_flux_yfaces": nxz * min(ny, 16),
-                 "elastic_yslabs": nxz * min(ny, 12)}
-        prof_keys = {"elastic_fused": ("elastic_fused (middle tiles)", "elastic_fused (edge tiles)"),
-                     "elastic_flux_yfaces": ("elastic_flux_batch (y faces)",), "elastic_yslabs": ("elastic_yslabs_ext",)}
+        cells = {"elastic_fused": nxz * ny}
+        prof_keys = {"elastic_fused": ("elastic_fused_step",)}
     else:
         inner = max(0, nx - 12) * max(0, ny - 12) * max(0, nz - 12)
         cells = {"elastic_interior": inner, "elastic_flux": nxz * ny, "elastic_boundary": 0,

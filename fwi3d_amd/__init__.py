@@ -316,12 +316,11 @@ class Engine:
 
     def tune(self, ychunk=None, tx=None, graphs=None, fused=None, fchunk=None, overlap=None, echunk=None):
         """Tiling of the time-step kernels, graph replay of time loops, and the elastic /
-        VTI step form (fused, the default: the fused kernel over the planes 6 cells inside
-        the y faces; fchunk: its y planes per workgroup, 0 by grid size; overlap: 0 one
-        stream, 1 / 2 its y-face launches on a second stream from the step's start / from
-        the edge tiles on, 3 its edge tiles on a second stream beside the middle tiles;
-        echunk: y planes per workgroup of its side tiles, 0 by grid size) (fwi3d_tune). Results do not depend on the tiling, the overlap or
-        graph replay; the two elastic forms agree to rounding."""
+        VTI step form (fused, the default: one launch per step; fchunk / echunk: y planes per
+        workgroup of its middle / side tiles, 0 by grid size; overlap: second stream of the
+        several launches that forward runs with a snapshot store take, 0..3, see
+        include/fwi3d_hip.h) (fwi3d_tune). Results do not depend on the tiling or graph replay; the two
+        elastic forms agree to rounding."""
         if ychunk is not None:
             self._check(lib().fwi3d_tune(self._h, 0, int(ychunk)), "fwi3d_tune")
         if tx is not None:
@@ -364,7 +363,7 @@ class Engine:
         self._check(lib().fwi3d_profile(self._h, level), "fwi3d_profile")
 
     def profile_read(self, kernel=0):
-        """(milliseconds, launches) of kernel class 0 (interior time step), 1 (flux
+        """(milliseconds, launches) of kernel class 0 (interior or fused time step), 1 (flux
         pre-pass, elastic/VTI), 2 (boundary-shell time step) or 3 (z-slab time step,
         elastic/VTI)."""
         ms = C.c_double()

@@ -26,7 +26,7 @@
 
 struct fwi3d_batch {
     enum Cls { C_AINT, C_ASHELL, C_AINJ, C_EFLUX, C_EINT, C_ESHELL, C_EZS, C_EINJ, C_VFLUX, C_VINT, C_VSHELL, C_VZS,
-               C_VINJ, C_EXT, C_EFUSED, C_VFUSED, C_EFEDGE, C_VFEDGE, C_EYS, C_VYS, NCLS };
+               C_VINJ, C_EXT, C_EFUSED, C_VFUSED, C_EMID, C_VMID, C_EEDGE, C_VEDGE, C_EYS, C_VYS, NCLS };
     struct Shot {
         int id = -1;
         fwi3d::BShot d{};
@@ -95,9 +95,9 @@ size_t batch_shot_bytes(int phys, const Geom& g, const fwi3d_injector* inj, cons
     auto al = [](size_t x) { return (x + 255) / 256 * 256; };
     const int ncomp = phys == FWI3D_ACOUSTIC ? 1 : 3;
     const int nmf = phys == FWI3D_ACOUSTIC ? 2 : (phys == FWI3D_ELASTIC ? 3 : 7);
-    const int naux = phys == FWI3D_ACOUSTIC ? 0 : (phys == FWI3D_ELASTIC ? 7 : 9);
     const size_t n = (size_t)g.n;
-    return al(3 * ncomp * n * 4) + al(nmf * n * 4) + al(naux * n * 4) + al((size_t)(g.nz + g.nx + g.ny) * 4) +
+    const size_t aux = phys == FWI3D_ACOUSTIC ? 0 : aux_bytes(phys == FWI3D_VTI, g);
+    return al(3 * ncomp * n * 4) + al(nmf * n * 4) + al(aux) + al((size_t)(g.nz + g.nx + g.ny) * 4) +
            al(inj_bytes(inj)) + al(inj_bytes(ext));
 }
 
@@ -146,7 +146,7 @@ void batch_retile(fwi3d_batch* b, int yc) {
         BShot& d = sh.d;
         if (d.phys == FWI3D_ACOUSTIC) {
             sh.nblk[B::C_AINT] = tile_grid_yc(d.a, d.g, b->TX, true, yc);
-        } else if (!d.fused) {  // (the fused kernel keeps its own y chunk)
+        } else if (d.form == STEP_FLUX) {  // (the fused kernels keep their own y chunks)
             const bool e = d.phys == FWI3D_ELASTIC;
             sh.nblk[e ? B::C_EFLUX : B::C_VFLUX] = tile_grid_yc(d.ef, d.g, b->TX, false, yc);
             sh.nblk[e ? B::C_EINT : B::C_VINT] = tile_grid_yc(d.ei, d.g, b->TX, true, yc);
@@ -207,20 +207,19 @@ void batch_one_step(fwi3d_batch* b, StepIdx it) {
     auto go_on = [&](hipStream_t sq, int k, auto kern, dim3 blk) {
         if (b->cls_blocks[k] > 0) hipLaunchKernelGGL(kern, dim3(b->cls_blocks[k]), blk, 0, sq, T, batch_map(b, k), it);
     };
-    auto go = [&](int k, auto kern, int threads, dim3 blk) {
-        go_on(st, k, kern, blk);
-        (void)threads;
-    };
+    auto go = [&](int k, auto kern, int, dim3 blk) { go_on(st, k, kern, blk); };
     go(B::C_EXT, extract_batch, 128, dim3(128));
-    // When every elastic / VTI shot runs the fused step, its launches write disjoint points
-    // of next and read no output of each other: as in the single-shot step, the fused edge
-    // tiles run on the context's second stream beside the middle tiles (FWI3D_TUNE_OVERLAP
-    // 3), or the y-face launches (flux pass of the 8 planes at each y face, then the y
-    // slabs) beside the edge tiles (1, 2).
+    // The launches of multi-launch fused shots write disjoint points of next and read no output
+    // of each other: when no shot needs the whole flux pass, their edge tiles run on the
+    // context's second stream beside the other tiles (FWI3D_TUNE_OVERLAP 3), or their y-face
+    // launches (flux pass of the 8 planes at each y face, then the y slabs) beside the edge
+    // tiles (1, 2).
     fwi3d_ctx* c = b->c;
-    bool ovl = c->fused_overlap != 0;
+    bool ovl = false;
+    if (c->fused_overlap != 0)
+        for (const auto& sh : b->shots) ovl = ovl || (sh.d.phys != FWI3D_ACOUSTIC && sh.d.form == STEP_MULTI);
     for (const auto& sh : b->shots)
-        if (sh.d.phys != FWI3D_ACOUSTIC && !sh.d.fused) ovl = false;
+        if (sh.d.phys != FWI3D_ACOUSTIC && sh.d.form == STEP_FLUX) ovl = false;
     auto yflux = [&](hipStream_t sq) {
         if (b->TX == 8) {
             go_on(sq, B::C_EFLUX, elastic_flux_batch<8, false>, dim3(64, 8));
@@ -237,8 +236,8 @@ void batch_one_step(fwi3d_batch* b, StepIdx it) {
     if (edge_side) {
         HIP_OK(hipEventRecord(c->fork_ev, st));
         HIP_OK(hipStreamWaitEvent(c->side, c->fork_ev, 0));
-        go_on(c->side, B::C_EFEDGE, elastic_fused_batch<false, true>, dim3(FTHREADS));
-        go_on(c->side, B::C_VFEDGE, elastic_fused_batch<true, true>, dim3(FTHREADS));
+        go_on(c->side, B::C_EEDGE, elastic_multi_batch<false, true>, dim3(FTHREADS));
+        go_on(c->side, B::C_VEDGE, elastic_multi_batch<true, true>, dim3(FTHREADS));
         HIP_OK(hipEventRecord(c->join_ev, c->side));
     }
     if (b->TX == 8) {
@@ -250,8 +249,13 @@ void batch_one_step(fwi3d_batch* b, StepIdx it) {
         go(B::C_EINT, elastic_interior_batch<4, false>, 0, dim3(64, 4));
         go(B::C_VINT, elastic_interior_batch<4, true>, 0, dim3(64, 4));
     }
-    go(B::C_EFUSED, elastic_fused_batch<false, false>, 0, dim3(FTHREADS));
-    go(B::C_VFUSED, elastic_fused_batch<true, false>, 0, dim3(FTHREADS));
+    for (int k : {B::C_EFUSED, B::C_VFUSED}) {
+        if (b->cls_blocks[k] == 0) continue;
+        auto kern = k == B::C_EFUSED ? elastic_fused_step<false> : elastic_fused_step<true>;
+        hipLaunchKernelGGL(kern, dim3(b->cls_blocks[k]), dim3(FTHREADS), 0, st, T, batch_map(b, k), it, INT_MAX);
+    }
+    go(B::C_EMID, elastic_multi_batch<false, false>, 0, dim3(FTHREADS));
+    go(B::C_VMID, elastic_multi_batch<true, false>, 0, dim3(FTHREADS));
     if (edge_side) {
         yflux(st);
         go(B::C_EYS, elastic_yslabs_batch<false>, 0, dim3(256));
@@ -265,8 +269,8 @@ void batch_one_step(fwi3d_batch* b, StepIdx it) {
             go_on(c->side, B::C_VYS, elastic_yslabs_batch<true>, dim3(256));
             HIP_OK(hipEventRecord(c->join_ev, c->side));
         }
-        go(B::C_EFEDGE, elastic_fused_batch<false, true>, 0, dim3(FTHREADS));
-        go(B::C_VFEDGE, elastic_fused_batch<true, true>, 0, dim3(FTHREADS));
+        go(B::C_EEDGE, elastic_multi_batch<false, true>, 0, dim3(FTHREADS));
+        go(B::C_VEDGE, elastic_multi_batch<true, true>, 0, dim3(FTHREADS));
     }
     go(B::C_ASHELL, acoustic_boundary_batch, 0, dim3(256));
     go(B::C_ESHELL, elastic_boundary_batch<false>, 0, dim3(256));
@@ -416,11 +420,10 @@ int batch_add_impl(fwi3d_batch* b, int mode, int physics, const float* d_model, 
         const int ncomp = physics == FWI3D_ACOUSTIC ? 1 : 3;
         const int npar = physics == FWI3D_ACOUSTIC ? 2 : (physics == FWI3D_ELASTIC ? 3 : 6);
         const int nmf = physics == FWI3D_ACOUSTIC ? 2 : (physics == FWI3D_ELASTIC ? 3 : 7);
-        const int naux = physics == FWI3D_ACOUSTIC ? 0 : (physics == FWI3D_ELASTIC ? 7 : 9);
         char* p = (char*)mem;
         float* F = (float*)p;          p += al(3 * ncomp * n * 4);
         float* M = (float*)p;          p += al(nmf * n * 4);
-        float* aux = (float*)p;        p += al(naux * n * 4);
+        float* aux = (float*)p;        p += al(physics == FWI3D_ACOUSTIC ? 0 : aux_bytes(physics == FWI3D_VTI, g));
         float* tp = (float*)p;         p += al((size_t)(g.nz + g.nx + g.ny) * 4);
         char* pinj = p;                p += al(inj_bytes(inj));
         char* pext = p;
@@ -491,19 +494,22 @@ int batch_add_impl(fwi3d_batch* b, int mode, int physics, const float* d_model, 
             d.nshell_blk = (d.nshell_pts + 255) / 256;
             s.nblk[grp == 1 ? B::C_ESHELL : B::C_VSHELL] = 0;  // the edges run in the slab class
             s.nblk[grp == 1 ? B::C_EZS : B::C_VZS] = zslab_tiles(d.zs, g) + 3 * d.nshell_blk;
-            if (c->use_fused) {
-                // the single-shot path's plan with the context's fused y chunks, not the
-                // autotuned ones: those are timed for one shot alone (a VTI shot's edge tiles
-                // in 4 long chunks, fewer workgroups than CUs beside its middle tiles, made
-                // the 32-shot batch 1.3x slower). The y chunks do not change a result bit.
-                (void)fchunk;
-                (void)echunk;
-                const FusedPlan P = fused_plan(d, g, TX, yc, c->fused_chunk, c->fused_echunk);
+            d.form = step_form(c, mode == 1);
+            if (d.form != STEP_FLUX)
+                for (int k : {B::C_EFLUX, B::C_VFLUX, B::C_EINT, B::C_VINT, B::C_EZS, B::C_VZS}) s.nblk[k] = 0;
+            // the single-shot path's plan with the context's fused y chunks, not the autotuned
+            // ones, which are timed for one shot alone. The y chunks do not change a result bit.
+            (void)fchunk;
+            (void)echunk;
+            if (d.form == STEP_FUSED) {
+                fused_plan(d, g, c->fused_chunk, c->fused_echunk);
+                fused_tables(st, vti, A, aux, d.ft);
+                s.nblk[grp == 1 ? B::C_EFUSED : B::C_VFUSED] = fused_workgroups(d.ft);
+            } else if (d.form == STEP_MULTI) {
+                const MultiPlan P = multi_plan(d, g, TX, yc, 0, 0);
                 s.nblk[grp == 1 ? B::C_EFLUX : B::C_VFLUX] = P.nflux;
-                s.nblk[grp == 1 ? B::C_EINT : B::C_VINT] = 0;
-                s.nblk[grp == 1 ? B::C_EFUSED : B::C_VFUSED] = P.nfused;
-                s.nblk[grp == 1 ? B::C_EFEDGE : B::C_VFEDGE] = P.nfedge;
-                s.nblk[grp == 1 ? B::C_EZS : B::C_VZS] = 0;
+                s.nblk[grp == 1 ? B::C_EMID : B::C_VMID] = P.nfused;
+                s.nblk[grp == 1 ? B::C_EEDGE : B::C_VEDGE] = P.nfedge;
                 s.nblk[grp == 1 ? B::C_EYS : B::C_VYS] = P.nslab;
             }
             s.nblk[grp == 1 ? B::C_EINJ : B::C_VINJ] = 3 * d.ninj_blk;
@@ -616,22 +622,6 @@ long long fwi3d_batch_snap_footprint(int physics, int nx, int ny, int nz, int nt
     }
 }
 
-// Batches whose fused elastic / VTI steps run on two streams and that hold 3 Mi cells or
-// more launch their steps directly, as single shots of that size do: replayed from a
-// captured graph, the two-stream step of the 32 VTI shots of the batched configuration
-// took 7.01 against 6.44 ms launched directly.
-bool batch_launch_directly(const fwi3d_batch* b) {
-    if (b->c->fused_overlap == 0) return false;
-    bool fused = false;
-    long long cells = 0;
-    for (const auto& sh : b->shots) {
-        if (sh.d.phys != FWI3D_ACOUSTIC && !sh.d.fused) return false;
-        fused = fused || sh.d.fused;
-        cells += (long long)sh.d.g.nx * sh.d.g.ny * sh.d.g.nz;
-    }
-    return fused && cells >= (3LL << 20);
-}
-
 int fwi3d_batch_step(fwi3d_batch* b, int nsteps, int* nactive) {
     if (!b) return FWI3D_EINVAL;
     fwi3d_ctx* c = b->c;
@@ -651,7 +641,7 @@ int fwi3d_batch_step(fwi3d_batch* b, int nsteps, int* nactive) {
             // a window of steps with no host work (no gradient shot, no tuning, no departure
             // before its last step) replays the captured graph; the last step of the window
             // may be a departure step, handled below
-            int quiet = tuning || !c->use_graphs || batch_launch_directly(b) ? 0 : nsteps - q;
+            int quiet = tuning || !c->use_graphs ? 0 : nsteps - q;
             for (const auto& sh : b->shots) {
                 if (sh.mode != 0) quiet = 0;
                 quiet = std::min(quiet, sh.d.t0 + sh.d.nt - 1 - b->it + 1);

@@ -9,8 +9,15 @@
 #include "acoustic.hpp"
 #include "elastic.hpp"
 #include "fused.hpp"
+#include "fused_multi.hpp"
+
+#include <type_traits>
 
 namespace fwi3d {
+
+// Forms of an elastic / VTI step: flux / interior / slab kernels, the fused kernel, or the
+// fused kernels of several launches.
+enum StepForm { STEP_FLUX = 0, STEP_FUSED = 1, STEP_MULTI = 2 };
 
 struct BShot {
     int phys;       // FWI3D_ACOUSTIC, FWI3D_ELASTIC or FWI3D_VTI
@@ -25,12 +32,13 @@ struct BShot {
     float* rcv;
     int nshell_blk;  // shell workgroups of one component (256 points each)
     int nshell_pts;  // shell points computed by the shell kernel (elastic / VTI: the edges and
-                     // corners; with the fused kernel the edges of the y slabs only)
+                     // corners)
     ZSlabTiles zs;   // elastic / VTI: tiling of the slab kernel (z slabs, then the side slabs)
-    int fused;       // elastic / VTI: the fused kernel updates the planes [6, ny-6), the slab
-                     // launch only the y slabs (side tiles and edges), the flux pass ef
-                     // covers the 8 planes at each y face
-    FusedTiles ft;   // tiling of the fused kernel
+    int form;        // elastic / VTI: STEP_FLUX, STEP_FUSED or STEP_MULTI
+    FusedTiles ft;   // one-launch fused step: tiling and boundary data
+    multi::FusedTiles mt;  // multi-launch fused step: tiling of the planes [6, ny-6); the slab
+                           // launch covers only the y slabs (side tiles and edges), the flux
+                           // pass ef the 8 planes at each y face
     int ninj_blk;    // injection workgroups of one component (256 targets each)
     int next_blk;    // extraction workgroups of one component (128 receivers)
 };
@@ -99,16 +107,17 @@ __global__ __launch_bounds__(256) void acoustic_boundary_batch(const BShot* __re
 }
 
 
-// Receivers of the single shot T[0] at local step k (they read curr, which no kernel of
-// the step writes), 256 per workgroup, component-major.
-__device__ __forceinline__ void extract_block256(const BShot& S, int l, int k) {
-    const int nb = (S.E.npts + 255) / 256;
-    const int r = (l % nb) * 256 + threadIdx.y * blockDim.x + threadIdx.x;  // 256 x 1 or 64 x 4 threads
+// Receivers of a single shot at local step k (they read curr, which no kernel of the step
+// writes), N (the workgroup's threads) per workgroup, component-major.
+template <int N>
+__device__ __forceinline__ void extract_block(const BShot& S, int l, int k) {
+    const int nb = (S.E.npts + N - 1) / N;
+    const int r = (l % nb) * N + threadIdx.y * blockDim.x + threadIdx.x;
     if (r >= S.E.npts) return;
     const float* curr = S.F + (long long)((k + 1) % 3) * S.nf;
     extract_one(curr, S.g, S.E, S.rcv, S.nt, k, r, l / nb);
 }
-__host__ __device__ inline int extract_blocks256(int npts, int ncomp) { return ncomp * ((npts + 255) / 256); }
+__host__ __device__ inline int extract_blocks(int npts, int ncomp, int n) { return ncomp * ((npts + n - 1) / n); }
 
 // Single-shot acoustic step in one launch of 64 x 4 threads per workgroup (the interior's
 // TX = 4 tile): the nint interior tiles (XCD-remapped among themselves), then the nshell
@@ -120,7 +129,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void a
     if (k < 0 || k > T[0].nt - 2) return;
     const int b = blockIdx.x;
     if (b >= nint + nshell) {
-        extract_block256(T[0], b - nint - nshell, k);
+        extract_block<256>(T[0], b - nint - nshell, k);
         return;
     }
     AcuArgs A = T[0].a;
@@ -140,7 +149,7 @@ __global__ __launch_bounds__(256) void acoustic_boundary_ext(const BShot* __rest
     const int k = it.value() - T[0].t0;
     if (k < 0 || k > T[0].nt - 2) return;
     if (L >= nshell) {
-        extract_block256(T[0], L - nshell, k);
+        extract_block<256>(T[0], L - nshell, k);
         return;
     }
     AcuArgs A = T[0].a;
@@ -178,12 +187,68 @@ __global__ __launch_bounds__(64 * TX) __attribute__((amdgpu_waves_per_eu(4))) vo
     elastic_interior_tile<TX, VTI>(A, [&] { return l; });
 }
 
-// Fused step over the planes [6, ny-6) (fused.hpp), 512 threads per workgroup: the
+// The whole elastic / VTI step of a shot (fused.hpp): workgroups of 512 threads, one tile
+// and y chunk (or y face) each, then (single-shot path) the receivers of the step from
+// workgroup nmain on. 4 waves per SIMD: two workgroups per CU hide each other's barriers.
+template <bool VTI>
+__global__ __launch_bounds__(FTHREADS) __attribute__((amdgpu_waves_per_eu(4))) void elastic_fused_step(
+    const BShot* __restrict__ T, BMap m, StepIdx it, int nmain) {
+    __shared__ FusedSmem<VTI> smem;
+    const int s = m.shot_of(blockIdx.x);
+    const int k = it.value() - T[s].t0;
+    if (k < 0 || k > T[s].nt - 2) return;
+    const int l = blockIdx.x - m.first(s);
+    if (l >= nmain) {
+        extract_block<FTHREADS>(T[s], l - nmain, k);
+        return;
+    }
+    const FusedTiles& FT = T[s].ft;
+    int cls, e;
+    if (!fused_item(FT, l, cls, e)) return;
+    EArgs A = T[s].ef;
+    bshot_rotate(A, T[s], k);
+    const int ntz = FT.ntz, ntx = FT.ntx;
+    using Yes = std::true_type;
+    using No = std::false_type;
+    if (cls == FC_YFACE) {
+        const int per = ntz * ntx, r = e % per, tz = r % ntz, tx = r / ntz, part = e / per;  // part: face, row half
+        const bool xe = tx == 0 || tx == ntx - 1, ze = tz == 0 || tz == ntz - 1;
+        auto run = [&](auto x, auto z) {
+            FusedTile<VTI, decltype(x)::value, decltype(z)::value>(A, FT, smem, tz, tx).yface(part >= 2, (part & 1) * 3);
+        };
+        if (!xe && !ze) run(No{}, No{});
+        else if (!ze) run(Yes{}, No{});
+        else if (!xe) run(No{}, Yes{});
+        else run(Yes{}, Yes{});
+        return;
+    }
+    auto march = [&](auto x, auto z, int tz, int tx, int per) {
+        const int ya = FT.ya + (e / per) * FT.chunk[cls], yb = min(FT.yb, ya + FT.chunk[cls]);
+        FusedTile<VTI, decltype(x)::value, decltype(z)::value>(A, FT, smem, tz, tx).march(ya, yb);
+    };
+    if (cls == FC_MID) {
+        const int per = fused_middle_tiles(ntz, ntx);
+        march(No{}, No{}, 1 + (e % per) % (ntz - 2), 1 + (e % per) / (ntz - 2), per);
+    }
+    if (cls == FC_SIDE) {
+        const int per = fused_side_tiles(ntz, ntx), q = fused_side_tile(e % per, ntz, ntx), tz = q & 0xffff, tx = q >> 16;
+        const bool xe = tx == 0 || tx == ntx - 1, ze = tz == 0 || tz == ntz - 1;
+        if (xe && ze) march(Yes{}, Yes{}, tz, tx, per);  // (an axis of one tile)
+        else if (xe) march(Yes{}, No{}, tz, tx, per);
+        else march(No{}, Yes{}, tz, tx, per);
+    }
+    if (cls == FC_CORNER) {
+        const int per = fused_corner_tiles(ntz, ntx), q = fused_corner_tile(e % per, ntz, ntx);
+        march(Yes{}, Yes{}, q & 0xffff, q >> 16, per);
+    }
+}
+
+// Fused step over the planes [6, ny-6) (fused_multi.hpp), 512 threads per workgroup: the
 // middle tiles (EDGE false) or the edge tiles of each y chunk (EDGE true).
 template <bool VTI, bool EDGE>
-__global__ __launch_bounds__(FTHREADS) __attribute__((amdgpu_waves_per_eu(VTI ? (EDGE ? 2 : 3) : (EDGE ? 2 : 4)))) void elastic_fused_batch(
+__global__ __launch_bounds__(FTHREADS) __attribute__((amdgpu_waves_per_eu(VTI ? (EDGE ? 2 : 3) : (EDGE ? 2 : 4)))) void elastic_multi_batch(
     const BShot* __restrict__ T, BMap m, StepIdx it) {
-    __shared__ FusedSmem<VTI> smem;
+    __shared__ multi::FusedSmem<VTI> smem;
     // XCD-contiguous workgroups (neighbouring tiles share halo lines in one L2): measured
     // 125 against 232 us for the x-edge tiles at 200^3 with the dispatch order.
     const int L = xcd_remap(blockIdx.x, gridDim.x);
@@ -192,7 +257,7 @@ __global__ __launch_bounds__(FTHREADS) __attribute__((amdgpu_waves_per_eu(VTI ? 
     if (k < 0 || k > T[s].nt - 2) return;
     EArgs A = T[s].ef;
     bshot_rotate(A, T[s], k);
-    const FusedTiles& FT = T[s].ft;
+    const multi::FusedTiles& FT = T[s].mt;
     const int l = L - m.first(s);
     if (EDGE) {
         // the side tiles first, then the corner tiles in their shorter y chunks
@@ -202,11 +267,11 @@ __global__ __launch_bounds__(FTHREADS) __attribute__((amdgpu_waves_per_eu(VTI ? 
         const int e = side ? l : l - ns, q = side ? per : ncor;
         const int tzx = side ? fused_side_tile(e % q, FT.ntz, FT.ntx) : fused_corner_tile(e % q, FT.ntz, FT.ntx);
         const int yc = side ? FT.sychunk : FT.cychunk, ya = FT.ya + (e / q) * yc;
-        elastic_fused_tile<VTI, true, true>(A, FT, tzx & 0xffff, tzx >> 16, ya, min(FT.yb, ya + yc), smem);
+        multi::elastic_fused_tile<VTI, true, true>(A, FT, tzx & 0xffff, tzx >> 16, ya, min(FT.yb, ya + yc), smem);
     } else {
         const int mz = FT.ntz - 2, per = mz * (FT.ntx - 2);
         const int r = l % per, ya = FT.ya + (l / per) * FT.ychunk;
-        elastic_fused_tile<VTI, false, false>(A, FT, 1 + r % mz, 1 + r / mz, ya, min(FT.yb, ya + FT.ychunk), smem);
+        multi::elastic_fused_tile<VTI, false, false>(A, FT, 1 + r % mz, 1 + r / mz, ya, min(FT.yb, ya + FT.ychunk), smem);
     }
 }
 
@@ -250,7 +315,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void e
     if (k < 0 || k > T[0].nt - 2) return;
     const int nb = T[0].nshell_blk;
     if (L >= 3 * nb) {
-        extract_block256(T[0], L - 3 * nb, k);
+        extract_block<256>(T[0], L - 3 * nb, k);
         return;
     }
     EArgs A = T[0].ef;
@@ -308,7 +373,7 @@ __global__ __launch_bounds__(256) void elastic_edges_slabs_ext(const BShot* __re
     }
     const int e = L - nslab, nb = T[0].nshell_blk;
     if (e >= 3 * nb) {
-        extract_block256(T[0], e - 3 * nb, k);
+        extract_block<256>(T[0], e - 3 * nb, k);
         return;
     }
     elastic_boundary_block<VTI>(A, e % nb, e / nb, T[0].nshell_pts);
@@ -342,7 +407,7 @@ __global__ __launch_bounds__(256) void elastic_edges_slabs_batch(const BShot* __
     elastic_boundary_block<VTI>(A, e % nb, e / nb, T[s].nshell_pts);
 }
 
-// Single-shot path with the fused kernel: the y-slab side tiles and edges (nslab
+// Single-shot path with the multi-launch fused step: the y-slab side tiles and edges (nslab
 // workgroups), then the receiver extraction of the same step. A kernel of its own, so
 // its code holds only these tiles (the instruction cache is the limit of the slab code).
 template <bool VTI>
@@ -352,7 +417,7 @@ __global__ __launch_bounds__(256) void elastic_yslabs_ext(const BShot* __restric
     if (k < 0 || k > T[0].nt - 2) return;
     const int L = blockIdx.x;
     if (L >= nslab) {
-        extract_block256(T[0], L - nslab, k);
+        extract_block<256>(T[0], L - nslab, k);
         return;
     }
     EArgs A = T[0].ef;

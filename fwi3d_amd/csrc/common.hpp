@@ -44,7 +44,17 @@ __device__ __forceinline__ GAS T* gas(T* p) { return (GAS T*)p; }
 __device__ __forceinline__ float gld(const float* base, unsigned i) {
     return *(const GAS float*)((const GAS char*)gas(base) + (i << 2));
 }
+// (byte offset, below 2^32)
+__device__ __forceinline__ float4 gld4(const float4* base, unsigned off) {
+    typedef float V4 __attribute__((ext_vector_type(4)));
+    const V4 v = *(const GAS V4*)((const GAS char*)gas((const char*)base) + off);
+    return make_float4(v.x, v.y, v.z, v.w);
+}
 __device__ __forceinline__ void gst(float* base, unsigned i, float v) { *(GAS float*)((GAS char*)gas(base) + (i << 2)) = v; }
+
+// A value that is the same in every lane, in a scalar register (floating-point results of
+// uniform operands are formed by vector instructions and would hold a vector register).
+__device__ __forceinline__ float uniform(float v) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v))); }
 
 // S and H weights (the closure rows are compile-time constants, below).
 __constant__ float c_sat_s[4];

@@ -79,7 +79,7 @@ struct fwi3d_ctx {
     std::vector<char> shot1_host;
     fwi3d::DevBuf shot1_dev;
     hipStream_t stream = nullptr;
-    // second stream of the fused elastic step (the y-face launches run on it beside the
+    // second stream of the multi-launch fused step (the y-face launches run on it beside the
     // fused tiles; default priority) and the fork / join events between the two
     hipStream_t side = nullptr;
     hipEvent_t fork_ev = nullptr, join_ev = nullptr;
@@ -117,14 +117,14 @@ struct fwi3d_ctx {
     // time loops without host work between steps replay a captured graph of several steps
     // (fwi3d_tune FWI3D_TUNE_GRAPHS); the counter the graph's kernels read the step from
     bool use_graphs = true;
-    // elastic / VTI steps: the fused kernel over the planes [6, ny-6) (fwi3d_tune
-    // FWI3D_TUNE_FUSED, default on) and its y chunk (FWI3D_TUNE_FCHUNK, 0: by grid size)
+    // elastic / VTI steps: the fused kernel (fwi3d_tune FWI3D_TUNE_FUSED, default on) and the y
+    // chunks of its middle and side tiles (FWI3D_TUNE_FCHUNK, FWI3D_TUNE_ECHUNK; 0: by grid size)
     bool use_fused = true;
     int fused_chunk = 0;
-    int fused_echunk = 0;  // y chunk of its side tiles (FWI3D_TUNE_ECHUNK, 0: fused_chunk's)
-    // launches of the fused step on the second stream (FWI3D_TUNE_OVERLAP): 0 none, 1 the
-    // y faces from the start of the step, 2 the y faces from the edge tiles on, 3 the edge
-    // tiles from the start of the step
+    int fused_echunk = 0;
+    // launches of the multi-launch fused step on the second stream (FWI3D_TUNE_OVERLAP): 0
+    // none, 1 the y faces from the start of the step, 2 the y faces from the edge tiles on, 3
+    // the edge tiles from the start of the step
     int fused_overlap = 3;
     fwi3d::DevBuf stepctr;
     std::vector<hipGraphExec_t> graph_execs;  // instantiated in the current call, freed after it

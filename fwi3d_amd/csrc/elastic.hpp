@@ -49,7 +49,7 @@ struct EArgs {
     // y-march tiling: tiles of 64 (z) x TX (x) x ychunk (y) from the corner (org, org, org);
     // the y march of the last chunk stops at yend. ysplit (flux pass only): two chunks,
     // the 8 planes at each y face (the planes the slab and edge kernels read fluxes from
-    // when the fused kernel updates the planes between them)
+    // in the multi-launch fused step)
     int ychunk, ntz, ntx, nyc, org, yend, ysplit;
 };
 

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -372,11 +373,86 @@ int zslab_tiles(ZSlabTiles& Z, const Geom& g) {
 // and corners (edge_point's enumeration).
 int shell_edge_count(const Geom& g) { return edge_count(6, g.nx, g.ny, g.nz); }
 
-// Elastic / VTI step with the fused kernel (fused.hpp): its tiling over the planes
-// [6, ny-6); the flux pass (d.ef) over the 8 planes at each y face, or the whole grid
-// when ny < 16; the slab launch over the y slabs: side tiles, then the y-slab points
-// within 6 cells of an x or z face (the first part of edge_point's enumeration).
-struct FusedPlan {
+// ---- elastic / VTI step with the fused kernel (fused.hpp)
+
+// Step form of a propagation: for a forward run that fills a snapshot store the multi-launch
+// fused step, whose rounding the codes of 16-bit stores have (fused_multi.hpp); FP32 stores
+// too, since the traces do not depend on the store's format.
+int step_form(const fwi3d_ctx* c, bool fwd_snap) {
+    if (!c->use_fused) return STEP_FLUX;
+    return fwd_snap ? STEP_MULTI : STEP_FUSED;
+}
+
+// Bytes of the flux buffer of a shot, which the fused step uses for its boundary tables and
+// dt^2 / rho instead (more than the fluxes on grids a few tens of points wide).
+size_t flux_bytes(bool vti, const Geom& g) { return (size_t)(vti ? 9 : 7) * g.n * sizeof(float); }
+size_t fused_bytes(bool vti, const Geom& g) { return closure_sizes(vti, g).total() * sizeof(float4) + (size_t)g.n * sizeof(float); }
+size_t aux_bytes(bool vti, const Geom& g) { return std::max(flux_bytes(vti, g), fused_bytes(vti, g)); }
+
+// Fill the boundary data of the fused step in `base` (fused_bytes).
+void fused_tables(hipStream_t st, bool vti, const EArgs& A, float* base, FusedTiles& F) {
+    const ClosureSizes cs = closure_sizes(vti, A.g);
+    F.tab = closure_tabs((float4*)base, cs);
+    float* rdt = (float*)((float4*)base + cs.total());
+    F.rdt = rdt;
+    const unsigned nb = (unsigned)std::min<size_t>(4096, (cs.total() / 2 + 255) / 256);
+    if (vti) hipLaunchKernelGGL(closure_tables<true>, dim3(nb), dim3(256), 0, st, A, (float4*)base, cs);
+    else hipLaunchKernelGGL(closure_tables<false>, dim3(nb), dim3(256), 0, st, A, (float4*)base, cs);
+    hipLaunchKernelGGL(rdt_field, dim3((unsigned)((A.g.n + 255) / 256)), dim3(256), 0, st, rdt, A.rho, A.dt2, A.g);
+}
+
+// Tiling of the fused step on a grid. A workgroup's time is about k (chunk + w) for its
+// class: w the iterations that fill its queues, k the cost of an iteration, a middle tile's
+// being 1 (side 1.05, corner 1.7; a y-face workgroup 9: fitted to sweeps). The y chunks are
+// those that give the march classes one time T, for the least estimated step: the work over
+// the slots (two workgroups per CU) and half of T for the ragged end, at least T and a y-face
+// workgroup's time where few workgroups leave slots idle. The best and worst elastic steps of
+// sweeps over (middle, side) chunks of 4..63 planes: 200^3 183 and 295 us, 256^3 306 and 423,
+// (ny, nx, nz) = (61, 75, 68) 33 and 181. fchunk / echunk set the middle / side tiles' by
+// hand (corners then take half of echunk).
+void fused_plan(BShot& d, const Geom& g, int fchunk, int echunk) {
+    d.form = STEP_FUSED;
+    FusedTiles& F = d.ft;
+    F.ntz = fused_tile_count(g.nz, FZ);
+    F.ntx = fused_tile_count(g.nx, FW);
+    F.ya = 6;
+    F.yb = g.ny - 6;
+    const int np = std::max(0, F.yb - F.ya);
+    const int tiles[FC_N] = {fused_corner_tiles(F.ntz, F.ntx), fused_side_tiles(F.ntz, F.ntx), 4 * F.ntz * F.ntx,
+                             fused_middle_tiles(F.ntz, F.ntx)};
+    constexpr double kCost[FC_N] = {1.7, 1.05, 9.0, 1.0}, kFill = 4.5, kSlots = 512, kYAlone = 10.0;
+    double best = 1e30;
+    int len[FC_N] = {1, 1, 1, 1};
+    for (int l = 1; l <= std::max(1, np); l++) {
+        const double T = l + kFill;
+        double work = kCost[FC_YFACE] * tiles[FC_YFACE];
+        int q[FC_N] = {1, 1, 1, 1};
+        for (int c : {FC_CORNER, FC_SIDE, FC_MID}) {
+            q[c] = std::max(1, std::min(std::max(np, 1), (int)(T / kCost[c] - kFill)));
+            work += tiles[c] * ((np + q[c] - 1) / q[c]) * kCost[c] * (q[c] + kFill);
+        }
+        const double cost = std::max({work / kSlots + 0.5 * T, T, kYAlone}) + 1e-3 * work / kSlots;
+        if (cost < best) {
+            best = cost;
+            std::copy(q, q + FC_N, len);
+        }
+    }
+    if (fchunk > 0) len[FC_MID] = fchunk;
+    if (echunk > 0) {
+        len[FC_SIDE] = echunk;
+        len[FC_CORNER] = std::max(4, echunk / 2);
+    }
+    for (int c = 0; c < FC_N; c++) {
+        F.chunk[c] = std::max(1, std::min(len[c], std::max(np, 1)));
+        F.n[c] = c == FC_YFACE ? tiles[c] : (np > 0 ? tiles[c] * ((np + F.chunk[c] - 1) / F.chunk[c]) : 0);
+    }
+}
+
+// ---- elastic / VTI step with the multi-launch fused kernels (fused_multi.hpp): their tiling
+// over the planes [6, ny-6); the flux pass (d.ef) over the 8 planes at each y face, or the
+// whole grid when ny < 16; the slab launch over the y slabs: side tiles, then the y-slab
+// points within 6 cells of an x or z face (the first part of edge_point's enumeration).
+struct MultiPlan {
     int nfused, nfedge, nflux, nslab;  // fused middle / edge workgroups, flux pass, slab launch
 };
 // Side-tile y chunk giving about `target` side workgroups (at least 8 planes: each chunk
@@ -387,10 +463,10 @@ int fused_side_chunk(int ntz, int ntx, int nyo, int target) {
     return std::max(8, (nyo + want - 1) / want);
 }
 
-FusedPlan fused_plan(BShot& d, const Geom& g, int TX, int ychunk, int fchunk, int echunk) {
-    FusedPlan P{};
-    d.fused = 1;
-    FusedTiles& F = d.ft;
+MultiPlan multi_plan(BShot& d, const Geom& g, int TX, int ychunk, int fchunk, int echunk) {
+    MultiPlan P{};
+    d.form = STEP_MULTI;
+    multi::FusedTiles& F = d.mt;
     F.ntz = fused_tile_count(g.nz, FZ);
     F.ntx = fused_tile_count(g.nx, FW);
     F.ya = 6;
@@ -632,7 +708,7 @@ void propagate_acoustic(fwi3d_ctx* c, bool adj, const float* d_model, const floa
     auto field = [&](int k) { return F + (long long)(k % 3) * n; };
     // one time step: receivers read curr, interior and shell write next, sources add to it
     // receivers are extracted by workgroups of the shell launch
-    const int ext_blk = (!adj && E.npts > 0) ? extract_blocks256(E.npts, 1) : 0;
+    const int ext_blk = (!adj && E.npts > 0) ? extract_blocks(E.npts, 1, 256) : 0;
     // with 4-row tiles the interior, shell and receivers share one launch, except when
     // every kernel is timed on its own (fwi3d_profile level 1)
     const bool one_launch = TX == 4 && nblk > 0 && !(c->prof && !c->prof_steps_only);
@@ -690,21 +766,27 @@ __global__ void vti_c11b_field(float* __restrict__ c11b, const float* __restrict
     if (i < n) c11b[i] = 2.f * (1.f + 2.f * eps[i]) * mu[i];
 }
 
-// One elastic/VTI time step: flux pre-pass, interior y-march, boundary shell.
-// The one-shot table T carries the flux pass's tiling (whole grid, nflux workgroups)
-// and the interior's (nint workgroups, 0 when the interior is empty).
-// next_blk: receiver-extraction workgroups launched with the shell (0: none this step).
-// One elastic/VTI time step with the fused kernel: fused planes, flux pass at the y
+// One elastic/VTI time step with the fused kernel, the receivers of the step in the last
+// ext_blk workgroups.
+template <bool VTI>
+void step_elastic_fused(fwi3d_ctx* c, const BShot* T, StepIdx it, const FusedTiles& F, int ext_blk) {
+    timed(c, 0, [&] {
+        const int n = fused_workgroups(F);
+        hipLaunchKernelGGL(elastic_fused_step<VTI>, dim3(n + ext_blk), dim3(FTHREADS), 0, c->stream, T, BMap{}, it, n);
+    });
+}
+
+// One elastic/VTI time step with the multi-launch fused kernels: fused planes, flux pass at the y
 // faces, y slabs with the receivers of the step.
 template <int TX, bool VTI>
-void step_elastic_fused(fwi3d_ctx* c, const BShot* T, StepIdx it, const FusedPlan& P, int next_blk) {
+void step_elastic_multi(fwi3d_ctx* c, const BShot* T, StepIdx it, const MultiPlan& P, int next_blk) {
     auto middle = [&](hipStream_t st) {
         if (P.nfused > 0)
-            hipLaunchKernelGGL((elastic_fused_batch<VTI, false>), dim3(P.nfused), dim3(FTHREADS), 0, st, T, BMap{}, it);
+            hipLaunchKernelGGL((elastic_multi_batch<VTI, false>), dim3(P.nfused), dim3(FTHREADS), 0, st, T, BMap{}, it);
     };
     auto edge = [&](hipStream_t st) {
         if (P.nfedge > 0)
-            hipLaunchKernelGGL((elastic_fused_batch<VTI, true>), dim3(P.nfedge), dim3(FTHREADS), 0, st, T, BMap{}, it);
+            hipLaunchKernelGGL((elastic_multi_batch<VTI, true>), dim3(P.nfedge), dim3(FTHREADS), 0, st, T, BMap{}, it);
     };
     // the y faces: flux pass of their 8 planes, then their 6 slab planes and the receivers
     auto yfaces = [&](hipStream_t st) {
@@ -755,6 +837,10 @@ void step_elastic_fused(fwi3d_ctx* c, const BShot* T, StepIdx it, const FusedPla
     HIP_OK(hipStreamWaitEvent(c->stream, c->join_ev, 0));
 }
 
+// One elastic/VTI time step of the flux / interior / slab form: flux pre-pass, interior
+// y-march, boundary shell. The one-shot table T carries the flux pass's tiling (whole grid,
+// nflux workgroups) and the interior's (nint workgroups, 0 when the interior is empty).
+// next_blk: receiver-extraction workgroups launched with the shell (0: none this step).
 template <int TX, bool VTI>
 void step_elastic(fwi3d_ctx* c, const BShot* T, StepIdx it, int nflux, int nint, int nshell_blk, int nzslab,
                   int next_blk) {
@@ -788,10 +874,15 @@ void propagate_elastic(fwi3d_ctx* c, bool vti, bool adj, const float* d_model, c
     const long long n = g.n;
     const int npar = vti ? 6 : 3;
     const int nmf = vti ? 7 : 3;  // device model fields (VTI adds c11b)
-    const int nT = vti ? 3 : 1;
     c->fields.ensure(9 * n * sizeof(float));
     c->model.ensure(nmf * n * sizeof(float));
-    c->aux.ensure((nT + 6) * n * sizeof(float));  // T (1 or 3), 6 shear fluxes
+    // the flux buffer, T (1 or 3) and 6 shear fluxes; or the fused step's boundary data. (A
+    // fixed workspace that holds the fluxes but not that data, on a narrow grid, runs the
+    // flux form.)
+    int form = step_form(c, !adj && par->sub > 0);
+    if (form == STEP_FUSED && c->aux.borrowed && c->aux.bytes < fused_bytes(vti, g)) form = STEP_FLUX;
+    const bool fused = form == STEP_FUSED;
+    c->aux.ensure(fused ? aux_bytes(vti, g) : flux_bytes(vti, g));
     float* F = c->fields.as<float>();
     float* Mf = c->model.as<float>();
     HIP_OK(hipMemsetAsync(F, 0, 9 * n * sizeof(float), c->stream));
@@ -846,9 +937,12 @@ void propagate_elastic(fwi3d_ctx* c, bool vti, bool adj, const float* d_model, c
     T1h.nshell_pts = shell_edge_count(g);
     T1h.nshell_blk = (T1h.nshell_pts + 255) / 256;
     const int nzslab = zslab_tiles(T1h.zs, g);
-    const bool fused = c->use_fused;
-    FusedPlan FP{};
-    if (fused) FP = fused_plan(T1h, g, TX, ychunk, fchunk, echunk);
+    MultiPlan MP{};
+    if (form == STEP_MULTI) MP = multi_plan(T1h, g, TX, ychunk, 0, 0);
+    if (fused) {
+        fused_plan(T1h, g, fchunk, echunk);
+        fused_tables(c->stream, vti, A, c->aux.as<float>(), T1h.ft);
+    }
     T1h.I = I; T1h.src = d_src; T1h.ninj_blk = nbi;
     T1h.E = E; T1h.rcv = d_rcv; T1h.next_blk = (E.npts + 127) / 128;
     const BShot* T1 = upload_shot1(c, T1h);
@@ -863,16 +957,21 @@ void propagate_elastic(fwi3d_ctx* c, bool vti, bool adj, const float* d_model, c
     // sources add to it (the batch kernels over the one-shot table: a batched shot runs
     // the same code)
     // receivers are extracted by workgroups of the shell launch
-    const int ext_blk = (!adj && E.npts > 0) ? extract_blocks256(E.npts, 3) : 0;
+    const int ext_blk = (!adj && E.npts > 0) ? extract_blocks(E.npts, 3, fused ? FTHREADS : 256) : 0;
     auto step = [&](StepIdx si) {
         timed(c, 4, [&] {
             if (fused) {
+                if (vti) step_elastic_fused<true>(c, T1, si, T1h.ft, ext_blk);
+                else step_elastic_fused<false>(c, T1, si, T1h.ft, ext_blk);
+                return;
+            }
+            if (form == STEP_MULTI) {
                 if (vti) {
-                    if (TX == 8) step_elastic_fused<8, true>(c, T1, si, FP, ext_blk);
-                    else step_elastic_fused<4, true>(c, T1, si, FP, ext_blk);
+                    if (TX == 8) step_elastic_multi<8, true>(c, T1, si, MP, ext_blk);
+                    else step_elastic_multi<4, true>(c, T1, si, MP, ext_blk);
                 } else {
-                    if (TX == 8) step_elastic_fused<8, false>(c, T1, si, FP, ext_blk);
-                    else step_elastic_fused<4, false>(c, T1, si, FP, ext_blk);
+                    if (TX == 8) step_elastic_multi<8, false>(c, T1, si, MP, ext_blk);
+                    else step_elastic_multi<4, false>(c, T1, si, MP, ext_blk);
                 }
                 return;
             }
@@ -891,15 +990,7 @@ void propagate_elastic(fwi3d_ctx* c, bool vti, bool adj, const float* d_model, c
     };
 
     if (!fwd_snap && !(adj && d_grad && sub > 0)) {
-        // no host work between steps: graph replay, except for fused two-stream steps of
-        // 3 Mi cells or more, launched directly. Replayed from a graph against launched
-        // directly, per step: 200^3 elastic 256 / 258 us (y faces on the second stream:
-        // 288 / 271), VTI 96 x 192 x 192 (nz, nx, ny) 236 / 214 us; below the threshold
-        // VTI 128^3 140 / 146 us, elastic 128^3 113 / 121 us.
-        if (fused && c->fused_overlap != 0 && (long long)g.nx * g.ny * g.nz >= (3LL << 20))
-            for (int it = 0; it < nt - 1; it++) step(StepIdx(it));
-        else
-            run_steps(c, 0, nt - 1, step);
+        run_steps(c, 0, nt - 1, step);  // no host work between steps
     } else {
         for (int it = 0; it < nt - 1; it++) {
             if (fwd_snap && it % sub == 0) snap_put(c->stream, ctx_snap(c), it / sub, field(it + 1));
@@ -1162,11 +1253,19 @@ int fwi3d_propagate_device_noalloc(fwi3d_ctx* c, int physics, int adj, const flo
         const int ncomp = ac ? 1 : 3, nmf = ac ? 2 : (physics == FWI3D_ELASTIC ? 3 : 7);
         const int naux = ac ? 0 : (physics == FWI3D_ELASTIC ? 7 : 9);
         auto al = [](size_t x) { return (x + 255) / 256 * 256; };
-        const size_t sz[7] = {al(3 * ncomp * n * 4), al(nmf * n * 4), al(naux * n * 4),
+        size_t sz[7] = {al(3 * ncomp * n * 4), al(nmf * n * 4), al(naux * n * 4),
                               al((size_t)(g.nz + g.nx + g.ny) * 4), al(inj_bytes(inj)),
                               adj ? 0 : al(inj_bytes(ext)), al(sizeof(BShot))};
         size_t total = 0;
         for (size_t x : sz) total += x;
+        // (the fused step's boundary data where it needs more than the fluxes and still fits)
+        if (!ac && c->use_fused && total <= kScratchBytes) {
+            const size_t more = al(aux_bytes(physics == FWI3D_VTI, g)) - sz[2];
+            if (total + more <= kScratchBytes) {
+                sz[2] += more;
+                total += more;
+            }
+        }
         REQUIRE(total <= kScratchBytes, "this shot needs " + std::to_string(total) + " bytes of workspace; the "
                                         "allocation-free entry point holds at most " + std::to_string(kScratchBytes) +
                                         " bytes (use fwi3d_propagate_device)");
@@ -1355,37 +1454,21 @@ int fwi3d_autotune(fwi3d_ctx* c, int physics, int nx, int ny, int nz, int steps,
                 if (t < best) { best = t; best_tx = tx; best_yc = yc; }
             }
         if (physics != FWI3D_ACOUSTIC && c->use_fused && ny > 12) {
-            // y chunk of the fused kernel's side tiles: about 0.6, 0.75, 1, 1.5, 2 or 2.5
-            // side workgroups per CU (the edge tiles run one workgroup per CU; beside the
-            // middle tiles, fewer edge workgroups than CUs can be fastest: 256^3 414
-            // against 451 us per step with 160 side workgroups). A chunk other
-            // than the grid-size rule's must be 3 % faster: the timings of 10-step runs
-            // vary by a few per cent, and a noisy pick cost a batch of three grids 10 %.
-            const int ntz = fused_tile_count(nz, FZ), ntx = fused_tile_count(nx, FW), nyo = ny - 12;
-            int tried[6], ntried = 0;
-            for (int target : {160, 192, 256, 384, 512, 640}) {
-                const int ec = fused_side_chunk(ntz, ntx, nyo, target);
-                if (std::find(tried, tried + ntried, ec) != tried + ntried) continue;
-                tried[ntried++] = ec;
-                c->fused_echunk = ec;
+            // y chunks of the fused kernel: the side tiles' and then the middle tiles' of the
+            // grid-size rule, scaled. Another chunk than the rule's must be 3 % faster: the
+            // timings of 10-step runs vary by a few per cent.
+            BShot probe{};
+            fused_plan(probe, make_geom(nx, ny, nz, 1.f, 1.f, 1.f), fc0, ec0);
+            for (double f : {0.6, 0.8, 1.25, 1.6}) {
+                c->fused_echunk = std::max(1, (int)(f * probe.ft.chunk[FC_SIDE]));
                 const double t = run(best_tx, best_yc);
-                if (t < 0.97 * best) { best = t; best_ec = ec; }
+                if (t < 0.97 * best) { best = t; best_ec = c->fused_echunk; }
             }
-            // middle-tile y chunk: one y chunk fewer or more per tile column than the
-            // grid-size rule's (the middle tiles share the CUs with the edge tiles)
             c->fused_echunk = best_ec > 0 ? best_ec : ec0;
-            if (fc0 <= 0) {
-                const int mid = fused_middle_tiles(ntz, ntx);
-                const int want = std::max(1, 512 / std::max(1, mid > 0 ? mid : ntz * ntx));
-                const int rule = std::max(8, (nyo + want - 1) / want);
-                for (int w : {want - 1, want + 1}) {
-                    if (w < 1) continue;
-                    const int fc = std::max(8, (nyo + w - 1) / w);
-                    if (fc == rule) continue;
-                    c->fused_chunk = fc;
-                    const double t = run(best_tx, best_yc);
-                    if (t < 0.97 * best) { best = t; best_fc = fc; }
-                }
+            for (double f : {0.6, 0.8, 1.25, 1.6}) {
+                c->fused_chunk = std::max(1, (int)(f * probe.ft.chunk[FC_MID]));
+                const double t = run(best_tx, best_yc);
+                if (t < 0.97 * best) { best = t; best_fc = c->fused_chunk; }
             }
         }
         restore();

@@ -126,7 +126,7 @@ int fwi3d_propagate_device_noalloc(fwi3d_ctx *ctx, int physics, int adj, const f
  * resets), enable=2 only whole time steps (class 4: fewer event records in the timed
  * work), 0 stops.
  * read() returns the summed milliseconds and launch count since the last enable of
- * kernel class `kernel`: 0 = the interior time-step kernel, 1 = the elastic/VTI flux
+ * kernel class `kernel`: 0 = the interior time-step kernel (or the fused one), 1 = the elastic/VTI flux
  * pre-pass, 2 = the boundary-shell time-step kernel (elastic/VTI: the shell's edges and
  * corners), 3 = the elastic/VTI slab kernel (the z slabs away from the x and y faces and
  * the x and y slabs away from the other faces), 4 = the whole time step. */
@@ -136,17 +136,16 @@ int fwi3d_propagate_device_noalloc(fwi3d_ctx *ctx, int physics, int adj, const f
  * FWI3D_TUNE_GRAPHS (default 1): time loops with no host work between steps (forward
  * propagation without snapshots, adjoint propagation without a gradient) replay a
  * captured hipGraph of 16 steps instead of launching each kernel.
- * FWI3D_TUNE_FUSED (default 1): elastic / VTI steps update the planes 6 cells inside the
- * y faces with the fused kernel (stresses and fluxes formed on chip; 0: the flux pass,
- * interior, slab and edge kernels over the whole grid). FWI3D_TUNE_FCHUNK: y planes per
- * workgroup of the fused kernel (0: chosen from the grid size). FWI3D_TUNE_OVERLAP
- * (default 3): the fused step's edge tiles run on a second stream of the context beside
- * its middle tiles, the y-face launches (their flux pass and slabs) after the middle
- * tiles (3); or the y-face launches run on the second stream, forked after the middle
- * tiles (2) or at the start of the step (1); or all on one stream (0). Results agree
- * to rounding between the two elastic forms and depend on none of the other settings.
- * FWI3D_TUNE_ECHUNK: y planes per workgroup of the fused kernel's side tiles (the tiles
- * at the x or z faces; 0: the middle tiles' chunk). */
+ * FWI3D_TUNE_FUSED (default 1): elastic / VTI steps run the fused kernel (one launch,
+ * stresses and fluxes formed on chip; 0: the flux pass, interior, slab and edge kernels).
+ * FWI3D_TUNE_FCHUNK: y planes per workgroup of the fused kernel's middle tiles,
+ * FWI3D_TUNE_ECHUNK of its side tiles (the tiles at the x or z faces; the corner tiles take
+ * half of it); 0: chosen from the grid size. Forward propagations that fill a
+ * snapshot store run the fused step as several launches, whose rounding the codes of 16-bit
+ * stores have; FWI3D_TUNE_OVERLAP is for these: the edge tiles run on a second stream of the
+ * context beside the middle tiles (3, the default), the y-face launches from the edge tiles
+ * on (2) or from the start of the step (1), or all on one stream (0). Results agree to
+ * rounding between the elastic forms and depend on none of the other settings. */
 enum fwi3d_tune_param {
     FWI3D_TUNE_YCHUNK = 0,
     FWI3D_TUNE_TX = 1,
@@ -159,9 +158,8 @@ enum fwi3d_tune_param {
 int fwi3d_tune(fwi3d_ctx *ctx, int param, int value);
 /* Autotuner (no counterpart in the reference): times `steps` time steps of the given
  * physics and grid on a synthetic model for every tile shape (TX 4 or 8, y chunk 4, 8,
- * 16 or 32, and for the fused elastic / VTI step the y chunk of its side tiles, about
- * 0.6 to 2.5 side workgroups per CU, and of its middle tiles, one chunk fewer or more
- * per tile column than the grid-size rule's; a chunk other than the rule's is kept when
+ * 16 or 32, and for the fused elastic / VTI step the y chunks of its side and of its middle
+ * tiles, 0.6 to 1.6 times the grid-size rule's; another chunk than the rule's is kept when
  * it is at least 3 % faster) with HIP events, keeps the fastest for that
  * physics and grid on the context
  * (used by propagate and by batch admission in preference to fwi3d_tune's settings) and

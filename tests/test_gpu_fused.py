@@ -175,3 +175,81 @@ def test_edge_chunks_identical(eng, physics):
     assert np.isfinite(ref).all() and np.abs(ref).max() > 0
     for k, v in out.items():
         assert np.array_equal(v, ref), k
+
+
+@pytest.mark.parametrize("physics", ["elastic", "vti"])
+@pytest.mark.parametrize("shape,case", [((12, 12, 12), "mixed"), ((12, 33, 64), "absorb-all"),
+                                        ((13, 17, 39), "free-all"), ((20, 56, 104), "mixed"),
+                                        ((19, 23, 32), "free+absorb+taper"), ((26, 16, 73), "absorb-all")])
+def test_fused_tile_classes_match_oracle(eng, physics, shape, case):
+    """The tile classes of the one-launch step at their limits: no plane between the y faces
+    (12 planes) or one, axes of one tile, two tiles (33, 39 along z; 17, 23 along x), and
+    middle tiles in every row and column of tiles (56 x 104); y chunks of 3 planes with
+    remainders. Tolerances as above: relative L2 of rounding over 40 steps."""
+    nt = 40
+    print(f"[fused classes {physics}] shape={shape} case={case} nt={nt}", flush=True)
+    got, (model, src, sloc, rloc, d, dt, cfg) = every_point(eng, physics, shape, case, nt=nt, fchunk=3)
+    oinj, oext = O.Injector(1, sloc, shape, d, (0, 0, 0)), O.Injector(0, rloc, shape, d, (0, 0, 0))
+    opar = O.make_par(nt, 0, dt, bc=cfg["bc"], taper=cfg["taper"])
+    want, _ = O.propagate(physics, model, src, oinj, oext, opar, d, s="f")
+    last = np.abs(got[:, :, -1] - want[:, :, -1]).max() / np.abs(want[:, :, -1]).max()
+    print(f"  rel L2 vs oracle f32 {rel(got, want):.2e}, worst point of the last sample {last:.2e}")
+    assert np.isfinite(got).all() and np.abs(want[:, :, -1]).max() > 0
+    assert rel(got, want) <= TRACE_TOL and last <= 10 * TRACE_TOL
+
+
+def test_narrow_grid_in_the_fixed_workspace(eng):
+    """On a narrow grid the fused step's boundary tables exceed the flux buffer: a shot that
+    fits the fixed workspace only with the flux buffer still runs there, by the flux form."""
+    import torch
+    shape, nt = (2280, 12, 64), 6
+    d = (0.01, 0.01, 0.01)
+    print(f"[narrow workspace] shape={shape}", flush=True)
+    dev = torch.device("cuda:0")
+    m = torch.stack([torch.full(shape, v, device=dev) for v in (8.0, 6.0, 2.3)]).contiguous()
+    src = torch.rand((6, 1, nt), generator=torch.Generator(device=dev).manual_seed(3), device=dev)
+    inj = F.Injector(1, np.array([[0.0513, 11.4013, 0.3013]], np.float32), shape, d)
+    ext = F.Injector(0, np.array([[0.0613, 11.4113, 0.2913]], np.float32), shape, d)
+    par = F.make_param(nt, 0.0008, bc=(1, 2, 2, 2, 2, 2))
+    out = []
+    for f in (eng.propagate_device, eng.propagate_device_noalloc):
+        r = torch.zeros((3, 1, nt), device=dev)
+        torch.cuda.synchronize()
+        f("elastic", m.data_ptr(), src.data_ptr(), r.data_ptr(), inj, ext, par, shape, d)
+        out.append(r.cpu().numpy())
+    assert np.abs(out[0]).max() > 0
+    assert rel(out[1], out[0]) <= 1e-5  # the two step forms agree to rounding
+
+
+@pytest.mark.parametrize("physics", ["elastic", "vti"])
+@pytest.mark.parametrize("shape,case", [((12, 12, 12), "mixed"), ((15, 20, 36), "absorb-all"),
+                                        ((16, 23, 33), "free-all"), ((30, 45, 104), "free+absorb+taper")])
+def test_store_forward_every_point_matches_oracle(eng, physics, shape, case):
+    """A forward run that fills a snapshot store takes the step of several launches:
+    every point against the oracle, on grids with the whole flux pass (ny < 16) and with the
+    y-face one, and bitwise the same on one and on two
+    streams and for every store format. Tolerances as above."""
+    nt = 40
+    print(f"[store {physics}] shape={shape} case={case} nt={nt}", flush=True)
+    model, src, sloc, _, d, dt = small_shot(physics, 1, shape=shape, nt=nt)
+    h = d[0]
+    iy, ix, iz = np.meshgrid(*(np.arange(n) for n in shape), indexing="ij")
+    rloc = np.stack([ix.ravel() * h, iy.ravel() * h, iz.ravel() * h], axis=1).astype(np.float32)
+    cfg = CASES[case]
+    inj, ext = F.Injector(1, sloc, shape, d), F.Injector(0, rloc, shape, d)
+    got = []
+    try:
+        for sp, ov in (("bf16", 0), ("bf16", 1), ("f32", 2), ("f16", 3)):
+            eng.tune(overlap=ov)
+            par = F.make_param(nt, dt, sub=4, bc=cfg["bc"], taper=cfg["taper"], snap_precision=sp)
+            got.append(eng.propagate(physics, model, src, inj, ext, par, d))
+    finally:
+        eng.tune(overlap=3)
+    oinj, oext = O.Injector(1, sloc, shape, d, (0, 0, 0)), O.Injector(0, rloc, shape, d, (0, 0, 0))
+    want, _ = O.propagate(physics, model, src, oinj, oext, O.make_par(nt, 0, dt, bc=cfg["bc"], taper=cfg["taper"]),
+                          d, s="f")
+    last = np.abs(got[0][:, :, -1] - want[:, :, -1]).max() / np.abs(want[:, :, -1]).max()
+    print(f"  rel L2 vs oracle f32 {rel(got[0], want):.2e}, worst point of the last sample {last:.2e}")
+    assert all(np.array_equal(g, got[0]) for g in got[1:])
+    assert np.isfinite(got[0]).all() and np.abs(want[:, :, -1]).max() > 0
+    assert rel(got[0], want) <= TRACE_TOL and last <= 10 * TRACE_TOL
