@@ -329,41 +329,4 @@ __device__ __forceinline__ void extract_one(const float* __restrict__ u3, const 
     gas(rcv)[(long long)(comp * I.npts + r) * nt + it] = acc;
 }
 
-// Imaging condition of nl_we_op_a::compute_gradients (we_op.cpp:1555-1605), FP64
-// accumulation. Snapshot views of slots itl-1, itl, itl+1 (a slot past the store has a
-// null base and reads as zero); branch: 0 first sample, 1 middle, 2 last. Gradients
-// use the unpadded reference layout.
-template <int FMT>
-__global__ void acoustic_grad(SnapView<FMT> fm, SnapView<FMT> fn, SnapView<FMT> fp, const float* __restrict__ adj,
-                              const float* __restrict__ K, Geom g, float sdt, int branch, double* __restrict__ gK,
-                              double* __restrict__ gB) {
-    const int iz = blockIdx.x * blockDim.x + threadIdx.x;
-    const int ix = blockIdx.y * blockDim.y + threadIdx.y;
-    const int iy = blockIdx.z;
-    if (iz >= g.nz || ix >= g.nx) return;
-    const int p = g.at(ix, iy, iz);
-    const float sn = fn.scale();
-    auto FN = [&](int i) { return fn.code(i); };
-    const float fx = d1_acc(FN, p, ix, g.nx, g.sx) * sn / g.dx;
-    const float fy = d1_acc(FN, p, iy, g.ny, g.sy) * sn / g.dy;
-    const float fz = d1_acc(FN, p, iz, g.nz, 1) * sn / g.dz;
-    const float ax = d1_point(adj, p, ix, g.nx, g.sx) / g.dx;
-    const float ay = d1_point(adj, p, iy, g.ny, g.sy) / g.dy;
-    const float az = d1_point(adj, p, iz, g.nz, 1) / g.dz;
-    const float dot = ax * fx + ay * fy + az * fz;
-    const float k = K[p];
-    const float fnv = fn.code(p) * sn;
-    const float fmv = fm.code(p) * fm.scale();
-    const float fpv = fp.p ? fp.code(p) * fp.scale() : 0.f;
-    float d2t;
-    if (branch == 1) d2t = fpv - 2.f * fnv + fmv;
-    else if (branch == 0) d2t = fpv - fnv;
-    else d2t = -2.f * fnv + fmv;
-    const float gk = 1.0f / (sdt * k * k) * adj[p] * d2t;
-    const float gb = (branch == 0 ? 0.5f : 1.0f) * sdt * dot;
-    const long long q = ((long long)iy * g.nx + ix) * g.nz + iz;
-    gK[q] -= (double)gk;
-    gB[q] += (double)gb;
-}
-
 }  // namespace fwi3d

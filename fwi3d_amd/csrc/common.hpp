@@ -210,17 +210,6 @@ __device__ __forceinline__ float sat_s(const float* __restrict__ u_, int p, int 
     return c_sat_s[0] * u[p] + c_sat_s[1] * u[p + inward] + c_sat_s[2] * u[p + 2 * inward] + c_sat_s[3] * u[p + 3 * inward];
 }
 
-// D1 (times h) at axis index i through an accessor f(offset) (snapshot views).
-template <class F>
-__device__ __forceinline__ float d1_acc(const F& f, int p, int i, int n, int s) {
-    if (i >= 4 && i < n - 4) return D1C1 * (f(p + s) - f(p - s)) + D1C2 * (f(p + 2 * s) - f(p - 2 * s));
-    const bool lo = i < 4;
-    const int base = lo ? p - i * s : p + (n - 1 - i) * s;
-    const int step = lo ? s : -s;
-    const float v = d1_rows(lo ? i : n - 1 - i, [&](int j) { return f(base + j * step); });
-    return lo ? v : -v;
-}
-
 // ------------------------------------------------------------------------------------
 // Snapshot store. FP32, or 16-bit codes (BF16 / FP16) of u / s with one scale per
 // snapshot, s = max|u| / 2^15: the largest value maps to 2^15, inside FP16's range,
@@ -241,10 +230,10 @@ struct SnapView {
     const void* p;           // slot base (null: a slot past the store, reads as zero)
     const unsigned* maxbits;  // the slot's max|u| as float bits (16-bit formats)
     __device__ float scale() const { return FMT == SNAP_F32 ? 1.f : __uint_as_float(*maxbits) / kSnapTop; }
-    __device__ float code(int i) const {
-        if (FMT == SNAP_F32) return ((const float*)p)[i];
-        if (FMT == SNAP_BF16) return bf16_val(((const unsigned short*)p)[i]);
-        return __half2float(((const __half*)p)[i]);
+    __device__ float code(unsigned i) const {
+        if (FMT == SNAP_F32) return gld((const float*)p, i);
+        const unsigned short h = *(const GAS unsigned short*)((const GAS char*)gas((const char*)p) + (i << 1));
+        return FMT == SNAP_BF16 ? bf16_val(h) : __half2float(__ushort_as_half(h));
     }
 };
 

@@ -992,108 +992,4 @@ __global__ void elastic_inject(float* __restrict__ out3, EArgs A, InjTab I, cons
     if (j < I.ntgt) elastic_inject_one<VTI>(out3, A, I, src, nt, it, mode, j, blockIdx.y);
 }
 
-// Imaging condition of nl_we_op_e / nl_we_op_vti ::compute_gradients
-// (we_op.cpp:488-565, 1108-1216) with FP64 accumulation. `lag` is the adjoint field
-// of the previous step (the reference uses the derivatives computed one step earlier);
-// `adj` the current adjoint field (rho term). Gradients in the unpadded layout.
-// Workgroups of 64 (z) x GTX (x) points of one y plane: the forward-field codes and the
-// lagged adjoint field of the tile and its 2-cell x / z halos are staged in LDS once, so
-// the interior x and z derivatives read on-chip values (closure rows and the y
-// derivatives read memory, as d1_acc / d1_point do; same arithmetic).
-constexpr int GTX = 4;  // 200^3 event: 472 us (8 x rows: 514, 16: 570; fewer workgroups hide less latency)
-template <bool VTI, int FMT>
-__global__ __launch_bounds__(64 * GTX) void elastic_grad(SnapView<FMT> fm, SnapView<FMT> fn, SnapView<FMT> fp,
-                                                    const float* __restrict__ adj, const float* __restrict__ lag, EArgs A,
-                                                    float sdt, int branch, double* __restrict__ gl, double* __restrict__ gm,
-                                                    double* __restrict__ gr) {
-    __shared__ float sf[3][GTX + 4][68], sl[3][GTX + 4][68];  // [component][x row from x0-2][z column from z0-2]
-    const Geom g = A.g;
-    const int lz = threadIdx.x, lx = threadIdx.y;
-    const int z0 = blockIdx.x * 64, x0 = blockIdx.y * GTX, iy = blockIdx.z;
-    const int iz = z0 + lz, ix = x0 + lx;
-    const int n3 = g.n;
-    const int pl = iy * g.sy;
-    const int p = pl + min(ix, g.nx - 1) * g.sx + min(iz, g.nz - 1);
-    HaloMap<GTX> H;
-    H.init(lx, lz, x0, z0, g.nx, g.nz, g.sx);
-#pragma unroll
-    for (int c = 0; c < 3; c++) {
-        sf[c][lx + 2][lz + 2] = fn.code(c * n3 + p);
-        sl[c][lx + 2][lz + 2] = lag[c * n3 + p];
-        if (H.has_x) {
-            sf[c][H.xrow][H.xcol] = fn.code(c * n3 + pl + H.xsrc);
-            sl[c][H.xrow][H.xcol] = lag[c * n3 + pl + H.xsrc];
-        }
-        if (H.has_z) {
-            sf[c][H.zrow][H.zcol] = fn.code(c * n3 + pl + H.zsrc);
-            sl[c][H.zrow][H.zcol] = lag[c * n3 + pl + H.zsrc];
-        }
-    }
-    __syncthreads();
-    if (iz >= g.nz || ix >= g.nx) return;
-    const bool inx = ix >= 4 && ix < g.nx - 4, inz = iz >= 4 && iz < g.nz - 4;
-    float F[3][3], Aj[3][3];  // [deriv axis][component]
-    const float sn = fn.scale();
-#pragma unroll
-    for (int c = 0; c < 3; c++) {
-        auto FN = [&](int i) { return fn.code(c * n3 + i); };
-        const float fx = inx ? D1C1 * (sf[c][lx + 3][lz + 2] - sf[c][lx + 1][lz + 2]) +
-                                   D1C2 * (sf[c][lx + 4][lz + 2] - sf[c][lx][lz + 2])
-                             : d1_acc(FN, p, ix, g.nx, g.sx);
-        const float fz = inz ? D1C1 * (sf[c][lx + 2][lz + 3] - sf[c][lx + 2][lz + 1]) +
-                                   D1C2 * (sf[c][lx + 2][lz + 4] - sf[c][lx + 2][lz])
-                             : d1_acc(FN, p, iz, g.nz, 1);
-        const float ax = inx ? D1C1 * (sl[c][lx + 3][lz + 2] - sl[c][lx + 1][lz + 2]) +
-                                   D1C2 * (sl[c][lx + 4][lz + 2] - sl[c][lx][lz + 2])
-                             : d1_point(lag + c * n3, p, ix, g.nx, g.sx);
-        const float az = inz ? D1C1 * (sl[c][lx + 2][lz + 3] - sl[c][lx + 2][lz + 1]) +
-                                   D1C2 * (sl[c][lx + 2][lz + 4] - sl[c][lx + 2][lz])
-                             : d1_point(lag + c * n3, p, iz, g.nz, 1);
-        F[0][c] = fx * sn / g.dx;
-        F[1][c] = d1_acc(FN, p, iy, g.ny, g.sy) * sn / g.dy;
-        F[2][c] = fz * sn / g.dz;
-        Aj[0][c] = ax / g.dx;
-        Aj[1][c] = d1_point(lag + c * n3, p, iy, g.ny, g.sy) / g.dy;
-        Aj[2][c] = az / g.dz;
-    }
-    // forward-field terms named as in the reference: temp[0..8]
-    const float t0 = F[0][0], t1 = F[1][1], t2 = F[2][2], t3 = F[0][2], t4 = F[2][0], t5 = F[0][1], t6 = F[1][0],
-                t7 = F[1][2], t8 = F[2][1];
-    const float w = branch == 0 ? 0.5f : 1.0f;
-    float gL, gM;
-    if (!VTI) {
-        gL = w * sdt * (Aj[0][0] + Aj[1][1] + Aj[2][2]) * (t0 + t1 + t2);
-        gM = w * sdt * ((Aj[2][0] + Aj[0][2]) * (t3 + t4) + (Aj[1][0] + Aj[0][1]) * (t5 + t6) +
-                        (Aj[2][1] + Aj[1][2]) * (t7 + t8) + 2.f * Aj[0][0] * t0 + 2.f * Aj[1][1] * t1 +
-                        2.f * Aj[2][2] * t2);
-    } else {
-        const float L = A.lam[p], U = A.mu[p], E = A.eps[p], C13 = A.c13[p], C66 = A.c66[p];
-        const float del = ((C13 + U) * (C13 + U) - (L + U) * (L + U)) / (2.f * (L + U) * (L + 2.f * U));
-        const float gam = (C66 - U) / (2.f * U);
-        const float v1 = sqrtf(2.f * (L + 2.f * U) * (L + U) * del + (L + U) * (L + U));
-        const float v2 = ((1.f + 2.f * del) * L + (1.f + 3.f * del) * U) / v1;
-        const float v3 = ((1.f + 3.f * del) * L + (1.f + 4.f * del) * U) / v1 - 1.f;
-        const float v4 = (Aj[0][0] + Aj[1][1]) * t2 + Aj[2][2] * (t0 + t1);
-        gL = w * sdt * ((1.f + 2.f * E) * (Aj[0][0] + Aj[1][1]) * (t0 + t1) + Aj[2][2] * t2 + v2 * v4);
-        gM = w * sdt * (2.f * (1.f + 2.f * E) * (Aj[0][0] * t0 + Aj[1][1] * t1) + 2.f * Aj[2][2] * t2 +
-                        4.f * (E - gam) * (Aj[0][0] * t1 + Aj[0][0] * t0) + (Aj[1][2] + Aj[2][1]) * (t7 + t8) +
-                        (Aj[0][2] + Aj[2][0]) * (t3 + t4) + (1.f + 2.f * gam) * (Aj[0][1] + Aj[1][0]) * (t5 + t6) +
-                        v3 * v4);
-    }
-    float rt = 0.f;
-    const float sm = fm.scale(), sp = fp.p ? fp.scale() : 0.f;
-#pragma unroll
-    for (int c = 0; c < 3; c++) {
-        const int qc = c * n3 + p;
-        const float fpv = fp.p ? fp.code(qc) * sp : 0.f;
-        const float fnv = fn.code(qc) * sn, fmv = fm.code(qc) * sm;
-        const float d2t = branch == 1 ? fpv - 2.f * fnv + fmv : (branch == 0 ? fpv - fnv : -fnv + fmv);
-        rt += adj[qc] * d2t;
-    }
-    const long long o = ((long long)iy * g.nx + ix) * g.nz + iz;
-    gl[o] += (double)gL;
-    gm[o] += (double)gM;
-    gr[o] += (double)(1.0f / sdt * rt);
-}
-
 }  // namespace fwi3d

@@ -21,6 +21,7 @@
 #include "elastic.hpp"
 #include "batch_kernels.hpp"
 #include "sbp_tables.hpp"
+#include "imaging.hpp"
 #include "snapshots.hpp"
 
 using namespace fwi3d;
@@ -617,13 +618,14 @@ void grad_event_acoustic(hipStream_t st, const SnapDesc& S, int itl, int nt, int
     const float sdt = (float)sub * dt;
     const int last = nt / sub;
     const int branch = (itl > 0 && itl < last) ? 1 : (itl == 0 ? 0 : 2);
-    dim3 grid((g.nz + 63) / 64, (g.nx + 3) / 4, g.ny);  // 64 z x 4 x rows per workgroup
+    const ImagingTiles T = imaging_tiles(g);
+    const dim3 grid(T.ntz * T.ntx * T.nyc);
     with_snap_fmt(S.fmt, [&](auto tag) {
         constexpr int FMT = decltype(tag)::value;
         // a slot past the store reads as zero (the reference dereferences a null slot there)
         const SnapView<FMT> fn = snap_view<FMT>(S, itl), fm = itl > 0 ? snap_view<FMT>(S, itl - 1) : fn,
                             fp = snap_view<FMT>(S, itl + 1);
-        hipLaunchKernelGGL(acoustic_grad<FMT>, grid, dim3(64, 4), 0, st, fm, fn, fp, adjf, M, g, sdt, branch, gK, gB);
+        hipLaunchKernelGGL(acoustic_grad<FMT>, grid, dim3(FTHREADS), 0, st, fm, fn, fp, adjf, M, g, T, sdt, branch, gK, gB);
     });
 }
 
@@ -635,16 +637,17 @@ void grad_event_elastic(hipStream_t st, bool vti, const SnapDesc& S, int itl, in
     const int last = nt / sub;
     const int branch = (itl > 0 && itl < last) ? 1 : (itl == 0 ? 0 : 2);
     const Geom& g = A.g;
-    dim3 grid((g.nz + 63) / 64, (g.nx + GTX - 1) / GTX, g.ny);  // 64 z x GTX x rows per workgroup
+    const ImagingTiles T = imaging_tiles(g);
+    const dim3 grid(T.ntz * T.ntx * T.nyc);
     with_snap_fmt(S.fmt, [&](auto tag) {
         constexpr int FMT = decltype(tag)::value;
         const SnapView<FMT> fn = snap_view<FMT>(S, itl), fm = itl > 0 ? snap_view<FMT>(S, itl - 1) : fn,
                             fp = snap_view<FMT>(S, itl + 1);
         if (vti)
-            hipLaunchKernelGGL((elastic_grad<true, FMT>), grid, dim3(64, GTX), 0, st, fm, fn, fp, adjf, lagf, A, sdt, branch,
+            hipLaunchKernelGGL((elastic_grad<true, FMT>), grid, dim3(FTHREADS), 0, st, fm, fn, fp, adjf, lagf, A, T, sdt, branch,
                                grad, grad + nunp, grad + 2 * nunp);
         else
-            hipLaunchKernelGGL((elastic_grad<false, FMT>), grid, dim3(64, GTX), 0, st, fm, fn, fp, adjf, lagf, A, sdt, branch,
+            hipLaunchKernelGGL((elastic_grad<false, FMT>), grid, dim3(FTHREADS), 0, st, fm, fn, fp, adjf, lagf, A, T, sdt, branch,
                                grad, grad + nunp, grad + 2 * nunp);
     });
 }
