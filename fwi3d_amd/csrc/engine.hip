@@ -589,12 +589,12 @@ void snap_put(hipStream_t st, const SnapDesc& S, int k, const float* u) {
         return;
     }
     void* dst = S.data + (size_t)k * ne * 2;
-    const unsigned grid = (unsigned)std::min<size_t>(2048, (ne / 4 + 255) / 256 + 1);
-    hipLaunchKernelGGL(snap_maxabs, dim3(grid), dim3(256), 0, st, u, mb, (long long)ne);
+    const dim3 grid(snap_blocks(ne));
+    hipLaunchKernelGGL(snap_maxabs, grid, dim3(256), 0, st, u, mb, (long long)ne);
     if (S.fmt == FWI3D_SNAP_BF16)
-        hipLaunchKernelGGL(snap_store<SNAP_BF16>, dim3(2048), dim3(256), 0, st, u, dst, (const unsigned*)mb, (long long)ne);
+        hipLaunchKernelGGL(snap_store<SNAP_BF16>, grid, dim3(256), 0, st, u, dst, (const unsigned*)mb, (long long)ne);
     else
-        hipLaunchKernelGGL(snap_store<SNAP_F16>, dim3(2048), dim3(256), 0, st, u, dst, (const unsigned*)mb, (long long)ne);
+        hipLaunchKernelGGL(snap_store<SNAP_F16>, grid, dim3(256), 0, st, u, dst, (const unsigned*)mb, (long long)ne);
 }
 
 template <int FMT>
