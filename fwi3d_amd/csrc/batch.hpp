@@ -26,7 +26,7 @@
 
 struct fwi3d_batch {
     enum Cls { C_AINT, C_ASHELL, C_AINJ, C_EFLUX, C_EINT, C_ESHELL, C_EZS, C_EINJ, C_VFLUX, C_VINT, C_VSHELL, C_VZS,
-               C_VINJ, C_EXT, C_EFUSED, C_VFUSED, C_EMID, C_VMID, C_EEDGE, C_VEDGE, C_EYS, C_VYS, NCLS };
+               C_VINJ, C_EXT, C_EFUSED, C_VFUSED, C_EMID, C_VMID, C_EEDGE, C_VEDGE, C_EYS, C_VYS, C_AFUSED, NCLS };
     struct Shot {
         int id = -1;
         fwi3d::BShot d{};
@@ -96,7 +96,7 @@ size_t batch_shot_bytes(int phys, const Geom& g, const fwi3d_injector* inj, cons
     const int ncomp = phys == FWI3D_ACOUSTIC ? 1 : 3;
     const int nmf = phys == FWI3D_ACOUSTIC ? 2 : (phys == FWI3D_ELASTIC ? 3 : 7);
     const size_t n = (size_t)g.n;
-    const size_t aux = phys == FWI3D_ACOUSTIC ? 0 : aux_bytes(phys == FWI3D_VTI, g);
+    const size_t aux = phys == FWI3D_ACOUSTIC ? acoustic_aux_bytes(g, inj) : aux_bytes(phys == FWI3D_VTI, g);
     return al(3 * ncomp * n * 4) + al(nmf * n * 4) + al(aux) + al((size_t)(g.nz + g.nx + g.ny) * 4) +
            al(inj_bytes(inj)) + al(inj_bytes(ext));
 }
@@ -145,7 +145,7 @@ void batch_retile(fwi3d_batch* b, int yc) {
     for (auto& sh : b->shots) {
         BShot& d = sh.d;
         if (d.phys == FWI3D_ACOUSTIC) {
-            sh.nblk[B::C_AINT] = tile_grid_yc(d.a, d.g, b->TX, true, yc);
+            if (d.form == STEP_FLUX) sh.nblk[B::C_AINT] = tile_grid_yc(d.a, d.g, b->TX, true, yc);
         } else if (d.form == STEP_FLUX) {  // (the fused kernels keep their own y chunks)
             const bool e = d.phys == FWI3D_ELASTIC;
             sh.nblk[e ? B::C_EFLUX : B::C_VFLUX] = tile_grid_yc(d.ef, d.g, b->TX, false, yc);
@@ -249,6 +249,9 @@ void batch_one_step(fwi3d_batch* b, StepIdx it) {
         go(B::C_EINT, elastic_interior_batch<4, false>, 0, dim3(64, 4));
         go(B::C_VINT, elastic_interior_batch<4, true>, 0, dim3(64, 4));
     }
+    if (b->cls_blocks[B::C_AFUSED] > 0)
+        hipLaunchKernelGGL(acoustic_fused_step, dim3(b->cls_blocks[B::C_AFUSED]), dim3(FTHREADS), 0, st, T,
+                           batch_map(b, B::C_AFUSED), it, 0);
     for (int k : {B::C_EFUSED, B::C_VFUSED}) {
         if (b->cls_blocks[k] == 0) continue;
         auto kern = k == B::C_EFUSED ? elastic_fused_step<false> : elastic_fused_step<true>;
@@ -423,7 +426,7 @@ int batch_add_impl(fwi3d_batch* b, int mode, int physics, const float* d_model, 
         char* p = (char*)mem;
         float* F = (float*)p;          p += al(3 * ncomp * n * 4);
         float* M = (float*)p;          p += al(nmf * n * 4);
-        float* aux = (float*)p;        p += al(physics == FWI3D_ACOUSTIC ? 0 : aux_bytes(physics == FWI3D_VTI, g));
+        float* aux = (float*)p;        p += al(physics == FWI3D_ACOUSTIC ? acoustic_aux_bytes(g, inj) : aux_bytes(physics == FWI3D_VTI, g));
         float* tp = (float*)p;         p += al((size_t)(g.nz + g.nx + g.ny) * 4);
         char* pinj = p;                p += al(inj_bytes(inj));
         char* pext = p;
@@ -470,6 +473,10 @@ int batch_add_impl(fwi3d_batch* b, int mode, int physics, const float* d_model, 
             s.nblk[B::C_ASHELL] = d.nshell_blk;
             s.nblk[B::C_AINJ] = d.ninj_blk;
             A.prev = F; A.curr = F + n; A.next = F + 2 * n;
+            if (step_form(c, mode == 1) == STEP_FUSED) {
+                for (int k : {B::C_AINT, B::C_ASHELL, B::C_AINJ}) s.nblk[k] = 0;
+                s.nblk[B::C_AFUSED] = acoustic_fused_plan(st, d, d_src, (char*)aux, c->tune_ychunk);
+            }
             if (d.I.ntgt > 0)
                 hipLaunchKernelGGL(acoustic_inject, dim3(d.ninj_blk), dim3(256), 0, st, F, A, d.I, d_src, d.nt, 0, 1);
         } else {

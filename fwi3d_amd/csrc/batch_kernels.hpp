@@ -7,6 +7,7 @@
 // propagate().
 #pragma once
 #include "acoustic.hpp"
+#include "acoustic_fused.hpp"
 #include "elastic.hpp"
 #include "fused.hpp"
 #include "fused_multi.hpp"
@@ -15,8 +16,9 @@
 
 namespace fwi3d {
 
-// Forms of an elastic / VTI step: flux / interior / slab kernels, the fused kernel, or the
-// fused kernels of several launches.
+// Forms of a step: flux / interior / slab kernels (acoustic: interior and shell, and the
+// injection in a launch of its own), the fused kernel, or the fused kernels of several launches
+// (elastic / VTI).
 enum StepForm { STEP_FLUX = 0, STEP_FUSED = 1, STEP_MULTI = 2 };
 
 struct BShot {
@@ -26,6 +28,8 @@ struct BShot {
     float* F;       // three wavefield sets, rotated as prev / curr / next
     Geom g;
     AcuArgs a;      // acoustic: interior tiling
+    AcuTiles at;    // acoustic one-launch step: tiling
+    InjMap im;      // its source map
     EArgs ef, ei;   // elastic / VTI: flux-pass tiling, interior tiling
     InjTab I, E;    // source injector, receiver extractor
     const float* src;
@@ -34,7 +38,7 @@ struct BShot {
     int nshell_pts;  // shell points computed by the shell kernel (elastic / VTI: the edges and
                      // corners)
     ZSlabTiles zs;   // elastic / VTI: tiling of the slab kernel (z slabs, then the side slabs)
-    int form;        // elastic / VTI: STEP_FLUX, STEP_FUSED or STEP_MULTI
+    int form;        // STEP_FLUX, STEP_FUSED or (elastic / VTI) STEP_MULTI
     FusedTiles ft;   // one-launch fused step: tiling and boundary data
     multi::FusedTiles mt;  // multi-launch fused step: tiling of the planes [6, ny-6); the slab
                            // launch covers only the y slabs (side tiles and edges), the flux
@@ -140,6 +144,43 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void a
     } else {
         acoustic_boundary_block(A, b - nint, T[0].nshell_pts);
     }
+}
+
+// Acoustic step in one launch: per shot, nmain workgroups of tiles, then those that form the
+// injection values of the following step. In a single-shot launch the last `next` workgroups
+// extract the receivers (they read curr, which no workgroup writes).
+__global__ __launch_bounds__(FTHREADS) __attribute__((amdgpu_waves_per_eu(6))) void acoustic_fused_step(
+    const BShot* __restrict__ T, BMap m, StepIdx it, int next) {
+    __shared__ AcuSmem smem;
+    const int nb = (int)gridDim.x - next;
+    const int L = (int)blockIdx.x < nb ? (m.shot ? xcd_remap(blockIdx.x, nb) : (int)blockIdx.x) : 0;
+    const int s = m.shot_of(L);
+    const int k = it.value() - T[s].t0;
+    if (k < 0 || k > T[s].nt - 2) return;
+    if ((int)blockIdx.x >= nb) {
+        extract_block<FTHREADS>(T[0], blockIdx.x - nb, k);
+        return;
+    }
+    AcuArgs A = T[s].a;
+    bshot_rotate(A, T[s], k);
+    const AcuTiles t = T[s].at;
+    const InjMap im = T[s].im;
+    const int nmain = t.ntz * t.ntx * t.nyc;
+    int l = L - m.first(s);
+    if (l < nmain) {
+        if (!m.shot) l = xcd_remap(l, nmain);
+        const int tz = l % t.ntz, tx = (l / t.ntz) % t.ntx;
+        if (tz == 0 || tz == t.ntz - 1 || tx == 0 || tx == t.ntx - 1)
+            acoustic_fused_tile<true>(A, t, T[s].I, im, k, l, smem);
+        else
+            acoustic_fused_tile<false>(A, t, T[s].I, im, k, l, smem);
+    } else if (k + 1 <= T[s].nt - 2) {
+        acoustic_inj_value(A, T[s].I, T[s].im, T[s].src, T[s].nt, k + 1, (l - nmain) * FTHREADS + threadIdx.x);
+    }
+}
+// The injection values of step 0.
+__global__ __launch_bounds__(FTHREADS) void acoustic_inj_first(AcuArgs A, InjTab I, InjMap M, const float* __restrict__ src, int nt) {
+    acoustic_inj_value(A, I, M, src, nt, 0, blockIdx.x * FTHREADS + threadIdx.x);
 }
 
 // Single-shot path: the shell's nshell workgroups, then the receiver extraction of the

@@ -652,6 +652,51 @@ void grad_event_elastic(hipStream_t st, bool vti, const SnapDesc& S, int itl, in
     });
 }
 
+// ---- one-launch acoustic step (acoustic_fused.hpp)
+
+// Bytes of its boundary tables and of the source map of an injector.
+size_t acoustic_aux_bytes(const Geom& g, const fwi3d_injector* inj) {
+    const size_t nw = ((size_t)g.n + 31) / 32, nc = (size_t)inj_nper(inj->kind) * inj->npts;
+    return acoustic_tables_bytes(g) + nw * 8 +
+           ((size_t)g.ny * fused_tile_count(g.nx, FW) * fused_tile_count(g.nz, FZ) + 2 + nc + 2 * nc) * 4;
+}
+
+// Plan the step of shot d and fill its tables, source map and first injection values in `base`
+// (acoustic_aux_bytes). Returns the workgroups of its launch.
+int acoustic_fused_plan(hipStream_t st, BShot& d, const float* src, char* base, int chunk) {
+    const Geom& g = d.g;
+    d.form = STEP_FUSED;
+    AcuTiles& T = d.at;
+    T = acoustic_tiles(g, chunk);
+    T.tab = acoustic_tabs((float4*)base, g);
+    const long long nf = 2LL * ((long long)g.ny * g.nx + (long long)g.ny * g.nz + (long long)g.nx * g.nz);
+    hipLaunchKernelGGL(acoustic_tables, dim3((unsigned)((nf + 255) / 256)), dim3(256), 0, st, d.a, T.tab);
+    int nblk = T.ntz * T.ntx * T.nyc;
+    d.im = InjMap{};
+    const InjTab& I = d.I;
+    if (I.ntgt > 0) {
+        const int nw = (int)((g.n + 31) / 32), nfl = g.ny * T.ntx * T.ntz;
+        uint2* mask = (uint2*)(base + acoustic_tables_bytes(g));
+        int* flag = (int*)(mask + nw);
+        int* count = flag + nfl;
+        int* perm = count + 2;
+        d.im.flag = flag;
+        d.im.mask = mask;
+        d.im.perm = perm;
+        d.im.nv = inj_nper(I.kind) * I.npts;
+        d.im.V = (float*)(perm + d.im.nv);
+        const dim3 bw((std::max(nw, nfl) + 255) / 256), bt((I.ntgt + 255) / 256), th(256);
+        hipLaunchKernelGGL(inj_map_clear, bw, th, 0, st, mask, nw, flag, nfl, count);
+        hipLaunchKernelGGL(inj_map_mark, bt, th, 0, st, mask, flag, T.ntz, T.ntx, I, g);
+        hipLaunchKernelGGL(inj_map_number, bw, th, 0, st, mask, nw, count);
+        hipLaunchKernelGGL(inj_map_list, bt, th, 0, st, (const uint2*)mask, I, g, perm);
+        const int nb = (d.im.nv + FTHREADS - 1) / FTHREADS;
+        hipLaunchKernelGGL(acoustic_inj_first, dim3(nb), dim3(FTHREADS), 0, st, d.a, I, d.im, src, d.nt);
+        nblk += nb;
+    }
+    return nblk;
+}
+
 void propagate_acoustic(fwi3d_ctx* c, bool adj, const float* d_model, const float* d_src, float* d_rcv,
                         const fwi3d_injector* inj, const fwi3d_injector* ext, double* d_grad, const fwi3d_param* par,
                         const Geom& g) {
@@ -696,6 +741,16 @@ void propagate_acoustic(fwi3d_ctx* c, bool adj, const float* d_model, const floa
     T1h.nshell_blk = (nshell + 255) / 256;
     T1h.I = I; T1h.src = d_src; T1h.ninj_blk = nbi;
     T1h.E = E; T1h.rcv = d_rcv; T1h.next_blk = (E.npts + 127) / 128;
+    // A forward run that fills a snapshot store keeps the interior / shell kernels, whose
+    // rounding the codes of 16-bit stores have (the traces do not depend on the store's format).
+    // So does a shot that fits a fixed workspace only without the tables.
+    const size_t aux = acoustic_aux_bytes(g, inj);
+    const bool fused = step_form(c, fwd_snap) == STEP_FUSED && !(c->aux.borrowed && c->aux.bytes < aux);
+    int nfused = 0;
+    if (fused) {
+        c->aux.ensure(aux);
+        nfused = acoustic_fused_plan(c->stream, T1h, d_src, c->aux.as<char>(), c->tune_ychunk);
+    }
     const BShot* T1 = upload_shot1(c, T1h);
 
     if (I.ntgt > 0)
@@ -709,14 +764,20 @@ void propagate_acoustic(fwi3d_ctx* c, bool adj, const float* d_model, const floa
     };
     // fields of local step k: prev = F[k % 3], curr = F[(k + 1) % 3] (the kernels' rotation)
     auto field = [&](int k) { return F + (long long)(k % 3) * n; };
-    // one time step: receivers read curr, interior and shell write next, sources add to it
-    // receivers are extracted by workgroups of the shell launch
-    const int ext_blk = (!adj && E.npts > 0) ? extract_blocks(E.npts, 1, 256) : 0;
-    // with 4-row tiles the interior, shell and receivers share one launch, except when
-    // every kernel is timed on its own (fwi3d_profile level 1)
+    // one time step: the fused launch, which injects too; or interior and shell (with the
+    // receivers' workgroups) in one launch with 4-row tiles, except when every kernel is timed on
+    // its own (fwi3d_profile level 1), and the injection
     const bool one_launch = TX == 4 && nblk > 0 && !(c->prof && !c->prof_steps_only);
+    const int ext_blk = (!adj && E.npts > 0) ? extract_blocks(E.npts, 1, fused ? FTHREADS : 256) : 0;
     auto step = [&](StepIdx si) {
         timed(c, 4, [&] {
+            if (fused) {
+                timed(c, 0, [&] {
+                    hipLaunchKernelGGL(acoustic_fused_step, dim3(nfused + ext_blk), dim3(FTHREADS), 0, c->stream, T1, BMap{},
+                                       si, ext_blk);
+                });
+                return;
+            }
             if (one_launch) {
                 hipLaunchKernelGGL(acoustic_step_ext, dim3(nblk + T1h.nshell_blk + ext_blk), dim3(64, 4), 0, c->stream,
                                    T1, si, nblk, T1h.nshell_blk);
@@ -731,7 +792,7 @@ void propagate_acoustic(fwi3d_ctx* c, bool adj, const float* d_model, const floa
                                    T1h.nshell_blk);
             });
         });
-        if (I.ntgt > 0)
+        if (I.ntgt > 0 && !fused)
             hipLaunchKernelGGL(acoustic_inject_batch, dim3(nbi), dim3(nthr), 0, c->stream, T1, BMap{}, si);
     };
 
@@ -1262,8 +1323,8 @@ int fwi3d_propagate_device_noalloc(fwi3d_ctx* c, int physics, int adj, const flo
         size_t total = 0;
         for (size_t x : sz) total += x;
         // (the fused step's boundary data where it needs more than the fluxes and still fits)
-        if (!ac && c->use_fused && total <= kScratchBytes) {
-            const size_t more = al(aux_bytes(physics == FWI3D_VTI, g)) - sz[2];
+        if (c->use_fused && total <= kScratchBytes) {
+            const size_t more = al(ac ? acoustic_aux_bytes(g, inj) : aux_bytes(physics == FWI3D_VTI, g)) - sz[2];
             if (total + more <= kScratchBytes) {
                 sz[2] += more;
                 total += more;
@@ -1393,9 +1454,10 @@ int fwi3d_autotune(fwi3d_ctx* c, int physics, int nx, int ny, int nz, int steps,
     long long n0[fwi3d_ctx::kProfClasses];
     std::copy(c->prof_ms, c->prof_ms + fwi3d_ctx::kProfClasses, ms0);
     std::copy(c->prof_n, c->prof_n + fwi3d_ctx::kProfClasses, n0);
+    const bool uf0 = c->use_fused;
     const int tx0 = c->tune_tx, yc0 = c->tune_ychunk, ec0 = c->fused_echunk, fc0 = c->fused_chunk;
     auto restore = [&] {
-        c->tune_tx = tx0; c->tune_ychunk = yc0; c->fused_echunk = ec0; c->fused_chunk = fc0;
+        c->use_fused = uf0; c->tune_tx = tx0; c->tune_ychunk = yc0; c->fused_echunk = ec0; c->fused_chunk = fc0;
         c->prof = prof0; c->prof_steps_only = steps_only0;
         std::copy(ms0, ms0 + fwi3d_ctx::kProfClasses, c->prof_ms);
         std::copy(n0, n0 + fwi3d_ctx::kProfClasses, c->prof_n);
@@ -1448,6 +1510,8 @@ int fwi3d_autotune(fwi3d_ctx* c, int physics, int nx, int ny, int nz, int steps,
             if (rc != FWI3D_OK) throw Err{rc, fwi3d::thread_error()};
             return c->prof_ms[4] / steps;  // whole time steps (the kernels overlap)
         };
+        // the acoustic fused step has its rule; the tiles are those of the interior kernels
+        if (physics == FWI3D_ACOUSTIC) c->use_fused = false;
         run(4, 8);  // warm-up
         int best_tx = 4, best_yc = 8, best_ec = 0, best_fc = 0;
         double best = 1e30;

@@ -156,3 +156,42 @@ def test_acoustic_every_point_matches_oracle(eng, shape, case):
     assert np.isfinite(got).all() and np.abs(want[:, :, -1]).max() > 0
     assert e <= TRACE_TOL
     assert last <= 10 * TRACE_TOL
+
+
+@pytest.mark.parametrize("shape,case", [((12, 12, 12), "mixed"), ((13, 16, 32), "absorb-all+taper"), ((17, 17, 33), "free-all"),
+                                        ((25, 23, 39), "mixed"), ((24, 24, 40), "free+absorb+taper"), ((26, 41, 72), "mixed")])
+@pytest.mark.parametrize("ychunk", [0, 5])
+def test_fused_step_every_point_matches_oracle(eng, shape, case, ychunk):
+    """The one-launch step at the edges of its tiles (16 x, 32 z points, chunks of planes): the
+    whole field at every step, with sources whose stencils overlap (one pair inside a tile, one
+    across a tile's edge, one at a face); and the same with the interior / shell kernels. The
+    tolerance is that of the traces; the worst point of the last sample within 10 times it."""
+    nt, dt = 60, 0.001
+    print(f"[acoustic fused] shape={shape} case={case} ychunk={ychunk}", flush=True)
+    model, _, _, _, d = small_shot(shape=shape, nt=nt)
+    ny, nx, nz = shape
+    h = d[0]
+    pts = [(0.5 * (nx - 1), 0.5 * (ny - 1), 0.4 * (nz - 1)), (min(nx - 1, 15.6), 0.3 * (ny - 1), min(nz - 1, 31.4)), (0.3, 0.2, 0.1)]
+    sloc = np.array([[x * h, y * h, z * h] for x, y, z in pts for _ in range(2)], np.float32)
+    sloc[1::2] += np.float32(0.6 * h) * np.sign((np.array([nx, ny, nz]) - 1) * h / 2 - sloc[1::2])
+    sloc = np.clip(sloc, 0, (np.array([nx, ny, nz], np.float32) - 1) * np.float32(h))
+    rng = np.random.default_rng(2)
+    src = (W.ricker(25.0, nt, dt)[None, None, :] * rng.uniform(0.5, 1.5, (1, len(sloc), 1))).astype(np.float32)
+    iy, ix, iz = np.meshgrid(*(np.arange(n) for n in shape), indexing="ij")
+    rloc = np.stack([ix.ravel() * h, iy.ravel() * h, iz.ravel() * h], axis=1).astype(np.float32)
+    cfg = CASES[case]
+    inj, ext = F.Injector(0, sloc, shape, d), F.Injector(0, rloc, shape, d)
+    par = F.make_param(nt, dt, bc=cfg["bc"], taper=cfg["taper"])
+    want, _ = O.propagate("acoustic", model, src, O.Injector(0, sloc, shape, d, (0, 0, 0)),
+                          O.Injector(0, rloc, shape, d, (0, 0, 0)), O.make_par(nt, 0, dt, bc=cfg["bc"], taper=cfg["taper"]),
+                          d, s="f")
+    assert np.abs(want[:, :, -1]).max() > 0
+    for fused in (True, False):
+        eng.tune(fused=fused, ychunk=ychunk)
+        try:
+            got = eng.propagate("acoustic", model, src, inj, ext, par, d)
+        finally:
+            eng.tune(fused=True, ychunk=0)
+        last = np.abs(got[:, :, -1] - want[:, :, -1]).max() / np.abs(want[:, :, -1]).max()
+        print(f"  fused={fused}: rel L2 vs oracle {rel(got, want):.2e}, worst point of the last sample {last:.2e}")
+        assert np.isfinite(got).all() and rel(got, want) <= TRACE_TOL and last <= 10 * TRACE_TOL
