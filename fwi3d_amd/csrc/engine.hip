@@ -565,7 +565,9 @@ void snap_begin(fwi3d_ctx* c, int physics, int ncomp, const fwi3d_param* par, co
     const size_t bytes = snap_store_bytes(slots, ncomp, g.n, par->snap_precision);
     c->snaps.ensure(bytes);
     c->snapsc.ensure((size_t)slots * sizeof(unsigned));
-    HIP_OK(hipMemsetAsync(c->snaps.p, 0, bytes, c->stream));
+    // slots past the last stored step, (nt-1)/sub, are never written and read as zero
+    const size_t slot = bytes / slots, written = (size_t)((par->nt - 1) / par->sub + 1) * slot;
+    if (written < bytes) HIP_OK(hipMemsetAsync(c->snaps.as<char>() + written, 0, bytes - written, c->stream));
     HIP_OK(hipMemsetAsync(c->snapsc.p, 0, (size_t)slots * sizeof(unsigned), c->stream));
     c->snap_slots = slots; c->snap_ncomp = ncomp; c->snap_n = g.n; c->snap_nt = par->nt; c->snap_sub = par->sub;
     c->snap_physics = physics; c->snap_fmt = par->snap_precision;
