@@ -91,8 +91,9 @@ KERNEL_CLASSES = {
     False: ((0, "elastic_interior"), (1, "elastic_flux"), (2, "elastic_boundary"), (3, "elastic_zslab")),
 }
 STEP_KERNEL = {
-    True: "elastic time step = one elastic_fused_step launch (all tiles and the receivers; HIP events around each "
-          "step on the engine stream)",
+    True: "elastic time step = one elastic_fused_step launch (all tiles and the receivers); in the forward run, which "
+          "fills the snapshot store, the fused middle and edge tiles, the y faces' flux pass and slabs on two streams "
+          "(HIP events around each step on the engine stream; traffic: the one-launch step's)",
     False: "elastic time step = elastic_flux + elastic_interior + elastic_boundary + elastic_zslab launches "
            "(HIP events around each step on the engine stream)",
 }
@@ -114,8 +115,8 @@ def traffic_profile(n):
 
 def kernel_rooflines(fused, nz, nx, ny, avg_us, n):
     """Per kernel class of the elastic step: the cells it handles, its algorithmic bytes
-    (48 B per cell it updates: u, prev, lambda, mu, rho read, next written), its launch time, achieved GB/s and fraction of 8 TB/s, and its measured HBM
-    bytes per launch from the committed PMC summary when there is one."""
+    (48 B per cell it updates: u, prev, lambda, mu, rho read, next written), its launch
+    time, achieved GB/s and fraction of 8 TB/s, and its measured HBM bytes per launch from the committed PMC summary when there is one."""
     nxz = nx * nz
     if fused:
         cells = {"elastic_fused": nxz * ny}
@@ -716,7 +717,8 @@ def main():
                     help="elastic / VTI steps with the flux, interior, slab and edge kernels (fwi3d_tune "
                          "FWI3D_TUNE_FUSED = 0) instead of the fused kernel")
     ap.add_argument("--overlap", type=int, default=None, choices=(0, 1, 2, 3),
-                    help="streams of the fused step (fwi3d_tune FWI3D_TUNE_OVERLAP; default: the library's, 3)")
+                    help="streams of the several launches of steps that fill a snapshot store (fwi3d_tune FWI3D_TUNE_OVERLAP; "
+                         "default: the library's, 3)")
     ap.add_argument("--workload", default="gradient", choices=("gradient", "acoustic", "lbfgs", "batch", "serve"),
                     help="gradient: elastic shot gradient (default); acoustic: 100^3 acoustic forward modelling; "
                          "lbfgs: 256^3 mixed-precision l-BFGS FWI; batch: 32 VTI shots on 3 grids, batched vs one at "

@@ -1,7 +1,9 @@
-// Acoustic variable-density kernels (gfx950).
+// Acoustic variable-density kernels (gfx950): the interior / shell form of the step, run by
+// forward propagations that fill a snapshot store (the one-launch form: acoustic_fused.hpp),
+// and the point sources and receivers of every form.
 //
 // One time step of nl_we_op_a::propagate (src/cpp/we_op.cpp:1662-1791) is two
-// launches that write disjoint points of `next` and only read curr/prev/model:
+// sets of workgroups that write disjoint points of `next` and only read curr/prev/model:
 //   acoustic_interior  points 6+ cells inside every face: D2(1/rho) along x, y, z
 //                      from an LDS x-z plane and a register queue along y, the
 //                      leapfrog update and the cos^2 taper;

@@ -132,12 +132,15 @@ int fwi3d_propagate_device_noalloc(fwi3d_ctx *ctx, int physics, int adj, const f
  * the x and y slabs away from the other faces), 4 = the whole time step. */
 /* Tiling of the y-marching time-step kernels, per context (no counterpart in the
  * reference; the tile shapes an autotuner picks): FWI3D_TUNE_YCHUNK = y planes per
- * workgroup (0: default 8), FWI3D_TUNE_TX = x rows per workgroup (4 or 8).
+ * workgroup (0: default 8; the one-launch acoustic step: by grid size), FWI3D_TUNE_TX = x
+ * rows per workgroup (4 or 8).
  * FWI3D_TUNE_GRAPHS (default 1): time loops with no host work between steps (forward
  * propagation without snapshots, adjoint propagation without a gradient) replay a
  * captured hipGraph of 16 steps instead of launching each kernel.
- * FWI3D_TUNE_FUSED (default 1): elastic / VTI steps run the fused kernel (one launch,
- * stresses and fluxes formed on chip; 0: the flux pass, interior, slab and edge kernels).
+ * FWI3D_TUNE_FUSED (default 1): a step is one launch (elastic / VTI: stresses and fluxes
+ * formed on chip; 0: the flux pass, interior, slab and edge kernels; acoustic: with its
+ * injection; 0, and forward runs that fill a snapshot store: interior and shell, then the
+ * injection).
  * FWI3D_TUNE_FCHUNK: y planes per workgroup of the fused kernel's middle tiles,
  * FWI3D_TUNE_ECHUNK of its side tiles (the tiles at the x or z faces; the corner tiles take
  * half of it); 0: chosen from the grid size. Forward propagations that fill a
