@@ -473,7 +473,7 @@ int batch_add_impl(fwi3d_batch* b, int mode, int physics, const float* d_model, 
             s.nblk[B::C_ASHELL] = d.nshell_blk;
             s.nblk[B::C_AINJ] = d.ninj_blk;
             A.prev = F; A.curr = F + n; A.next = F + 2 * n;
-            if (step_form(c, mode == 1) == STEP_FUSED) {
+            if (step_form(c, mode == 1, physics, g) == STEP_FUSED) {
                 for (int k : {B::C_AINT, B::C_ASHELL, B::C_AINJ}) s.nblk[k] = 0;
                 s.nblk[B::C_AFUSED] = acoustic_fused_plan(st, d, d_src, (char*)aux, c->tune_ychunk);
             }
@@ -501,7 +501,7 @@ int batch_add_impl(fwi3d_batch* b, int mode, int physics, const float* d_model, 
             d.nshell_blk = (d.nshell_pts + 255) / 256;
             s.nblk[grp == 1 ? B::C_ESHELL : B::C_VSHELL] = 0;  // the edges run in the slab class
             s.nblk[grp == 1 ? B::C_EZS : B::C_VZS] = zslab_tiles(d.zs, g) + 3 * d.nshell_blk;
-            d.form = step_form(c, mode == 1);
+            d.form = step_form(c, mode == 1, physics, g);
             if (d.form != STEP_FLUX)
                 for (int k : {B::C_EFLUX, B::C_VFLUX, B::C_EINT, B::C_VINT, B::C_EZS, B::C_VZS}) s.nblk[k] = 0;
             // the single-shot path's plan with the context's fused y chunks, not the autotuned

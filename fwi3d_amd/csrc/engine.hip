@@ -378,10 +378,14 @@ int shell_edge_count(const Geom& g) { return edge_count(6, g.nx, g.ny, g.nz); }
 
 // Step form of a propagation: for a forward run that fills a snapshot store the multi-launch
 // fused step, whose rounding the codes of 16-bit stores have (fused_multi.hpp); FP32 stores
-// too, since the traces do not depend on the store's format.
-int step_form(const fwi3d_ctx* c, bool fwd_snap) {
+// too, since the traces do not depend on the store's format. So does a grid whose boundary
+// coefficients exceed the 32-bit byte offsets of the one-launch steps (a face of 3.7 M points
+// and more for VTI, 11 M for the others).
+int step_form(const fwi3d_ctx* c, bool fwd_snap, int physics, const Geom& g) {
     if (!c->use_fused) return STEP_FLUX;
-    return fwd_snap ? STEP_MULTI : STEP_FUSED;
+    const ClosureSizes s = closure_sizes(physics == FWI3D_VTI, g);
+    const bool fits = std::max(s.zc, std::max(s.xc, s.yc)) * sizeof(float4) < (1ULL << 32);
+    return fwd_snap || !fits ? STEP_MULTI : STEP_FUSED;
 }
 
 // Bytes of the flux buffer of a shot, which the fused step uses for its boundary tables and
@@ -747,7 +751,7 @@ void propagate_acoustic(fwi3d_ctx* c, bool adj, const float* d_model, const floa
     // rounding the codes of 16-bit stores have (the traces do not depend on the store's format).
     // So does a shot that fits a fixed workspace only without the tables.
     const size_t aux = acoustic_aux_bytes(g, inj);
-    const bool fused = step_form(c, fwd_snap) == STEP_FUSED && !(c->aux.borrowed && c->aux.bytes < aux);
+    const bool fused = step_form(c, fwd_snap, FWI3D_ACOUSTIC, g) == STEP_FUSED && !(c->aux.borrowed && c->aux.bytes < aux);
     int nfused = 0;
     if (fused) {
         c->aux.ensure(aux);
@@ -945,7 +949,7 @@ void propagate_elastic(fwi3d_ctx* c, bool vti, bool adj, const float* d_model, c
     // the flux buffer, T (1 or 3) and 6 shear fluxes; or the fused step's boundary data. (A
     // fixed workspace that holds the fluxes but not that data, on a narrow grid, runs the
     // flux form.)
-    int form = step_form(c, !adj && par->sub > 0);
+    int form = step_form(c, !adj && par->sub > 0, vti ? FWI3D_VTI : FWI3D_ELASTIC, g);
     if (form == STEP_FUSED && c->aux.borrowed && c->aux.bytes < fused_bytes(vti, g)) form = STEP_FLUX;
     const bool fused = form == STEP_FUSED;
     c->aux.ensure(fused ? aux_bytes(vti, g) : flux_bytes(vti, g));

@@ -253,3 +253,32 @@ def test_store_forward_every_point_matches_oracle(eng, physics, shape, case):
     assert all(np.array_equal(g, got[0]) for g in got[1:])
     assert np.isfinite(got[0]).all() and np.abs(want[:, :, -1]).max() > 0
     assert rel(got[0], want) <= TRACE_TOL and last <= 10 * TRACE_TOL
+
+
+def test_wide_face_keeps_32bit_offsets(eng):
+    """The boundary coefficients of a VTI face of 3.8 M points pass 4 GiB: such a grid runs the
+    step of several launches, with the flux form's results near the far corner of the face
+    (rounding of a few steps: 1e-5, as test_fused_equals_unfused)."""
+    import torch
+    shape, nt, h = (12, 1920, 1984), 12, 0.01
+    print(f"[wide face] shape={shape}", flush=True)
+    dev = torch.device("cuda:0")
+    m = torch.stack([torch.full(shape, v, device=dev) for v in (8.0, 6.0, 2.3, 8.2, 0.1, 6.3)]).contiguous()
+    src = torch.rand((6, 1, nt), generator=torch.Generator(device=dev).manual_seed(5), device=dev)
+    x, z = (shape[1] - 4) * h, (shape[2] - 4) * h
+    inj = F.Injector(1, np.array([[x + 0.003, 0.023, z + 0.004]], np.float32), shape, (h, h, h))
+    ext = F.Injector(0, np.array([[x + 0.011, 0.013, z - 0.006], [x - 0.012, 0.041, z]], np.float32), shape, (h, h, h))
+    par = F.make_param(nt, 0.0008, bc=(1, 2, 2, 2, 2, 2))
+    out = []
+    try:
+        for fused in (True, False):
+            eng.tune(fused=fused)
+            r = torch.zeros((3, 2, nt), device=dev)
+            torch.cuda.synchronize()
+            eng.propagate_device("vti", m.data_ptr(), src.data_ptr(), r.data_ptr(), inj, ext, par, shape, (h, h, h))
+            torch.cuda.synchronize()
+            out.append(r.cpu().numpy())
+    finally:
+        eng.tune(fused=True)
+    assert np.isfinite(out[0]).all() and np.abs(out[1]).max() > 0
+    assert rel(out[0], out[1]) <= 1e-5
