@@ -120,13 +120,13 @@ __global__ __launch_bounds__(256) void acoustic_tables(AcuArgs A, AcuTabs T) {
 struct AcuTiles { int ntz, ntx, nyc, chunk; AcuTabs tab; };
 // Planes per workgroup: as few as keep the workgroups within one round of the chip (three per
 // CU), at most 6 (on large grids, where several rounds run anyway, 5 to 10 measured alike and
-// 3 and 16 slower). chunk > 0: by hand.
+// 3 and 16 slower). chunk > 0: by hand (any count: past ny it is the whole axis).
 inline AcuTiles acoustic_tiles(const Geom& g, int chunk) {
     AcuTiles T{};
     T.ntz = fused_tile_count(g.nz, FZ);
     T.ntx = fused_tile_count(g.nx, FW);
     const int fit = std::max(1, 768 / (T.ntz * T.ntx));
-    T.chunk = chunk > 0 ? chunk : std::min(6, (g.ny + fit - 1) / fit);
+    T.chunk = std::min(g.ny, chunk > 0 ? chunk : std::min(6, (g.ny + fit - 1) / fit));
     T.nyc = (g.ny + T.chunk - 1) / T.chunk;
     return T;
 }

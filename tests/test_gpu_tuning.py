@@ -110,3 +110,27 @@ def test_graph_replay_equals_eager(physics, nt):
     r_eager = fwd_traces(physics, nt, False)
     assert np.abs(r_eager).max() > 0
     assert np.array_equal(r_graph, r_eager)
+
+
+def test_acoustic_y_chunks_of_any_length():
+    """The y chunk of the one-launch acoustic step by hand: one plane, a remainder, the whole
+    axis (21 planes) and counts past it up to the largest int give the rule's bits."""
+    from fwi3d_amd import workloads as W
+    shape, nt, d = (21, 27, 70), 40, (0.01, 0.01, 0.01)
+    vp = (1.8 + 0.6 * W.smooth_random(shape, 4, 3)).astype(np.float32)
+    model, src = W.acoustic_convert(vp, W.gardner(vp)), W.ricker(25, nt, 0.001)[None, None, :].astype(np.float32)
+    inj = F.Injector(0, [[0.13, 0.1, 0.3]], shape, d)
+    ext = F.Injector(0, [[0.05 + 0.04 * i, 0.05 + 0.03 * j, 0.03] for i in range(4) for j in range(4)], shape, d)
+    par = F.make_param(nt, 0.001, sub=0, bc=(1, 2, 2, 2, 2, 2), taper=(0, 4, 4, 4, 4, 4))
+    out = {}
+    eng = F.Engine(0)
+    try:
+        for yc in (0, 1, 4, 21, 22, 2**31 - 1):
+            print(f"  y chunk {yc}", flush=True)
+            eng.tune(ychunk=yc)
+            out[yc] = eng.propagate("acoustic", model, src, inj, ext, par, d)
+    finally:
+        eng.close()
+    assert np.abs(out[0]).max() > 0
+    for yc, r in out.items():
+        assert np.array_equal(r, out[0]), yc
