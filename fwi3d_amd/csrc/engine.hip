@@ -946,11 +946,11 @@ void propagate_elastic(fwi3d_ctx* c, bool vti, bool adj, const float* d_model, c
     const int nmf = vti ? 7 : 3;  // device model fields (VTI adds c11b)
     c->fields.ensure(9 * n * sizeof(float));
     c->model.ensure(nmf * n * sizeof(float));
-    // the flux buffer, T (1 or 3) and 6 shear fluxes; or the fused step's boundary data. (A
+    // the flux buffer, T (1 or 3) and 6 shear fluxes; or the one-launch step's boundary data. (A
     // fixed workspace that holds the fluxes but not that data, on a narrow grid, runs the
-    // flux form.)
+    // several-launch step, which needs only the fluxes of the y faces.)
     int form = step_form(c, !adj && par->sub > 0, vti ? FWI3D_VTI : FWI3D_ELASTIC, g);
-    if (form == STEP_FUSED && c->aux.borrowed && c->aux.bytes < fused_bytes(vti, g)) form = STEP_FLUX;
+    if (form == STEP_FUSED && c->aux.borrowed && c->aux.bytes < fused_bytes(vti, g)) form = STEP_MULTI;
     const bool fused = form == STEP_FUSED;
     c->aux.ensure(fused ? aux_bytes(vti, g) : flux_bytes(vti, g));
     float* F = c->fields.as<float>();

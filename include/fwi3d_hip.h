@@ -116,7 +116,9 @@ int fwi3d_propagate_device(fwi3d_ctx *ctx, int physics, int adj, const float *d_
  * counterpart here); a shot whose buffers exceed the workspace is rejected with
  * FWI3D_EINVAL. Every call on one GPU shares that workspace: calls that overlap on the
  * same GPU (other contexts, other threads) race and must be serialized by the caller.
- * Returns after the work has completed; results equal fwi3d_propagate_device's. */
+ * Returns after the work has completed; results equal fwi3d_propagate_device's (to
+ * rounding where the workspace holds the shot but not the boundary coefficients of the
+ * one-launch step: such a shot takes the step of a forward run with a snapshot store). */
 int fwi3d_propagate_device_noalloc(fwi3d_ctx *ctx, int physics, int adj, const float *d_model, const float *d_src,
                                    float *d_rcv, const fwi3d_injector *inj, const fwi3d_injector *ext,
                                    const fwi3d_param *par, int nx, int ny, int nz, float dx, float dy, float dz);

@@ -221,6 +221,36 @@ def test_narrow_grid_in_the_fixed_workspace(eng):
     assert rel(out[1], out[0]) <= 1e-5  # the two step forms agree to rounding
 
 
+@pytest.mark.parametrize("physics,shape", [("acoustic", (6700, 12, 64)), ("elastic", (2280, 12, 64)),
+                                           ("vti", (1720, 12, 64))])
+def test_fixed_workspace_without_boundary_tables(eng, physics, shape):
+    """A shot that fits the fixed workspace only without the boundary coefficients takes the
+    step of a forward run with a snapshot store: the same kernels in the same order, so the
+    same bits."""
+    import torch
+    nt, d, rng = 24, (0.01, 0.01, 0.01), np.random.default_rng(8)
+    ny, nx, nz = shape
+    print(f"[workspace limit {physics}] shape={shape}", flush=True)
+    dev = torch.device("cuda:0")
+    vals = {"acoustic": (8.0, 0.4), "elastic": (8.0, 6.0, 2.3), "vti": (8.0, 6.0, 2.3, 8.2, 0.1, 6.3)}[physics]
+    ns, nc = (1, 1) if physics == "acoustic" else (6, 3)
+    m = torch.stack([torch.full(shape, v, device=dev) for v in vals]).contiguous()
+    src = torch.from_numpy(rng.standard_normal((ns, 1, nt)).astype(np.float32)).to(dev)
+    y = ny // 2 * 0.01  # (the y-face slabs are the same kernels in both of the other forms)
+    inj = F.Injector(0 if ns == 1 else 1, np.array([[0.0513, y, 0.3013]], np.float32), shape, d)
+    ext = F.Injector(0, np.array([[0.0613, y + 0.01, 0.2913], [0.02, y - 0.03, 0.05]], np.float32), shape, d)
+    out = []
+    for f, sub in ((eng.propagate_device, nt), (eng.propagate_device_noalloc, 0)):
+        r = torch.zeros((nc, 2, nt), device=dev)
+        torch.cuda.synchronize()
+        f(physics, m.data_ptr(), src.data_ptr(), r.data_ptr(), inj, ext,
+          F.make_param(nt, 0.0008, sub=sub, bc=(1, 2, 2, 2, 2, 2)), shape, d)
+        torch.cuda.synchronize()
+        out.append(r.cpu().numpy())
+    assert np.isfinite(out[0]).all() and np.abs(out[0]).max() > 0
+    assert np.array_equal(out[1], out[0])
+
+
 @pytest.mark.parametrize("physics", ["elastic", "vti"])
 @pytest.mark.parametrize("shape,case", [((12, 12, 12), "mixed"), ((15, 20, 36), "absorb-all"),
                                         ((16, 23, 33), "free-all"), ((30, 45, 104), "free+absorb+taper")])
