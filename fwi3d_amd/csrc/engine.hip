@@ -1060,7 +1060,14 @@ void propagate_elastic(fwi3d_ctx* c, bool vti, bool adj, const float* d_model, c
     };
 
     if (!fwd_snap && !(adj && d_grad && sub > 0)) {
-        run_steps(c, 0, nt - 1, step);  // no host work between steps
+        // no host work between steps: graph replay, except for the step of two streams (very wide
+        // faces only, so large grids), launched directly. Replayed against launched directly, per
+        // step: elastic 200^3 256 / 258 us (y faces on the second stream: 288 / 271), VTI 96 x 192
+        // x 192 (nz, nx, ny) 236 / 214 us.
+        if (form == STEP_MULTI && c->fused_overlap != 0)
+            for (int it = 0; it < nt - 1; it++) step(StepIdx(it));
+        else
+            run_steps(c, 0, nt - 1, step);
     } else {
         for (int it = 0; it < nt - 1; it++) {
             if (fwd_snap && it % sub == 0) snap_put(c->stream, ctx_snap(c), it / sub, field(it + 1));

@@ -312,3 +312,25 @@ def test_wide_face_keeps_32bit_offsets(eng):
         eng.tune(fused=True)
     assert np.isfinite(out[0]).all() and np.abs(out[1]).max() > 0
     assert rel(out[0], out[1]) <= 1e-5
+
+
+def test_two_stream_step_is_launched_directly(eng):
+    """The several-launch step without a store (wide faces) is not replayed from a graph: the
+    profile counts the y faces' flux pass of every step (a replayed window counts none of its
+    kernels)."""
+    import torch
+    shape, nt, h = (12, 1920, 1984), 35, 0.01  # two windows of 16 steps and a remainder
+    print(f"[two streams] shape={shape}", flush=True)
+    dev = torch.device("cuda:0")
+    m = torch.stack([torch.full(shape, v, device=dev) for v in (8.0, 6.0, 2.3, 8.2, 0.1, 6.3)]).contiguous()
+    src = torch.zeros((6, 1, nt), device=dev)
+    inj = F.Injector(1, np.array([[1.003, 0.053, 1.004]], np.float32), shape, (h, h, h))
+    ext = F.Injector(0, np.zeros((0, 3), np.float32), shape, (h, h, h))
+    torch.cuda.synchronize()
+    eng.profile(True)
+    try:
+        eng.propagate_device("vti", m.data_ptr(), src.data_ptr(), 0, inj, ext, F.make_param(nt, 0.0008), shape, (h, h, h))
+        n = eng.profile_read(1)[1]
+    finally:
+        eng.profile(False)
+    assert n == nt - 1
