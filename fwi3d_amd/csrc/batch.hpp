@@ -522,7 +522,7 @@ int batch_add_impl(fwi3d_batch* b, int mode, int physics, const float* d_model, 
                 fused_tables(st, vti, A, aux, d.ft);
                 s.nblk[grp == 1 ? B::C_EFUSED : B::C_VFUSED] = fused_workgroups(d.ft);
             } else if (d.form == STEP_MULTI) {
-                const MultiPlan P = multi_plan(d, g, TX, yc, 0, 0);
+                const MultiPlan P = multi_plan(d, g, TX, yc, c->fused_chunk, c->fused_echunk);
                 s.nblk[grp == 1 ? B::C_EFLUX : B::C_VFLUX] = P.nflux;
                 s.nblk[grp == 1 ? B::C_EMID : B::C_VMID] = P.nfused;
                 s.nblk[grp == 1 ? B::C_EEDGE : B::C_VEDGE] = P.nfedge;

@@ -1008,7 +1008,7 @@ void propagate_elastic(fwi3d_ctx* c, bool vti, bool adj, const float* d_model, c
     T1h.nshell_blk = (T1h.nshell_pts + 255) / 256;
     const int nzslab = zslab_tiles(T1h.zs, g);
     MultiPlan MP{};
-    if (form == STEP_MULTI) MP = multi_plan(T1h, g, TX, ychunk, 0, 0);
+    if (form == STEP_MULTI) MP = multi_plan(T1h, g, TX, ychunk, c->fused_chunk, c->fused_echunk);
     if (fused) {
         fused_plan(T1h, g, fchunk, echunk);
         fused_tables(c->stream, vti, A, c->aux.as<float>(), T1h.ft);

@@ -134,3 +134,31 @@ def test_acoustic_y_chunks_of_any_length():
     assert np.abs(out[0]).max() > 0
     for yc, r in out.items():
         assert np.array_equal(r, out[0]), yc
+
+
+def test_y_chunks_reach_forward_runs_with_a_store():
+    """FWI3D_TUNE_FCHUNK / ECHUNK tile the several-launch step of a store-filling forward run
+    too: with chunks of one plane each workgroup marches 5 planes for the one it updates (8 of
+    12 by the grid-size rule), three times the work on a grid that fills the chip."""
+    shape, nt, d = (160, 160, 160), 16, (0.01, 0.01, 0.01)
+    model = np.stack([np.full(shape, v, np.float32) for v in (8.0, 6.0, 2.3)])
+    src = np.ones((6, 1, nt), np.float32)
+    inj = F.Injector(1, [[0.8, 0.8, 0.8]], shape, d)
+    ext = F.Injector(0, [[0.7, 0.7, 0.7]], shape, d)
+    par = F.make_param(nt, 0.0008, sub=nt)
+    us, out = {}, {}
+    eng = F.Engine(0)
+    try:
+        for c in (0, 1):
+            eng.tune(fchunk=c, echunk=c)
+            for _ in range(2):  # (the first call warms up)
+                eng.profile(True, steps_only=True)
+                out[c] = eng.propagate("elastic", model, src, inj, ext, par, d)
+                ms, n = eng.profile_read(4)
+            us[c] = 1e3 * ms / n
+            eng.profile(False)
+    finally:
+        eng.close()
+    print(f"  us per step by the rule {us[0]:.0f}, one plane per chunk {us[1]:.0f}", flush=True)
+    assert np.array_equal(out[0], out[1])
+    assert us[1] > 1.5 * us[0]
