@@ -461,9 +461,8 @@ int batch_add_impl(fwi3d_batch* b, int mode, int physics, const float* d_model, 
         d.src = d_src;
         d.rcv = d_rcv;
         const float dt = par->dt;
-        int tx_tuned, yc, echunk, fchunk;  // the batch's launches share one TX; the y chunks are per shot
-        tiles_for(c, physics, g, tx_tuned, yc, echunk, fchunk);
-        if (b->force_yc > 0) yc = b->force_yc;
+        const fwi3d_ctx::Tiles tiles = tiles_for(c, physics, g);  // the batch's launches share one TX; the y chunks are per shot
+        const int yc = b->force_yc > 0 ? b->force_yc : tiles.ychunk;
         const int TX = b->TX;
         const int nshell = shell_count(6, g.nx, g.ny, g.nz);
         d.nshell_blk = (nshell + 255) / 256;
@@ -484,7 +483,7 @@ int batch_add_impl(fwi3d_batch* b, int mode, int physics, const float* d_model, 
             A.prev = F; A.curr = F + n; A.next = F + 2 * n;
             if (step_form(c, mode == 1, physics, g) == STEP_FUSED) {
                 for (int k : {B::C_AINT, B::C_ASHELL, B::C_AINJ}) s.nblk[k] = 0;
-                s.nblk[B::C_AFUSED] = acoustic_fused_plan(st, d, d_src, (char*)aux, c->tune_ychunk);
+                s.nblk[B::C_AFUSED] = acoustic_fused_plan(st, d, d_src, (char*)aux, tiles.achunk);
             }
             if (d.I.ntgt > 0)
                 hipLaunchKernelGGL(acoustic_inject, dim3(d.ninj_blk), dim3(256), 0, st, F, A, d.I, d_src, d.nt, 0, 1);
@@ -514,9 +513,8 @@ int batch_add_impl(fwi3d_batch* b, int mode, int physics, const float* d_model, 
             if (d.form != STEP_FLUX)
                 for (int k : {B::C_EFLUX, B::C_VFLUX, B::C_EINT, B::C_VINT, B::C_EZS, B::C_VZS}) s.nblk[k] = 0;
             // the single-shot path's plan with the context's fused y chunks, not the autotuned
-            // ones, which are timed for one shot alone. The y chunks do not change a result bit.
-            (void)fchunk;
-            (void)echunk;
+            // ones, which are timed for one shot alone (a VTI shot's edge tiles in 4 long chunks made
+            // a 32-shot batch 1.3x slower). The y chunks do not change a result bit.
             if (d.form == STEP_FUSED) {
                 fused_plan(d, g, c->fused_chunk, c->fused_echunk);
                 fused_tables(st, vti, A, aux, d.ft);

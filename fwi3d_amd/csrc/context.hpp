@@ -107,11 +107,13 @@ struct fwi3d_ctx {
     // tiling of the y-marching kernels (fwi3d_tune)
     int tune_ychunk = 0;  // y planes per workgroup (0: default 8)
     int tune_tx = 4;      // x rows per workgroup (4 or 8)
-    // tiles chosen by fwi3d_autotune per physics and grid (they take precedence there)
+    // tiles chosen by fwi3d_autotune per physics and grid (they take precedence there); a chunk
+    // of 0: the context's setting, or by grid size
     struct Tiles {
         int physics, nx, ny, nz, tx, ychunk;
-        int echunk;  // side-tile y chunk of the fused elastic / VTI kernel (0: by grid size)
-        int fchunk;  // its middle-tile y chunk (0: by grid size)
+        int echunk, fchunk;    // one-launch elastic / VTI step: side tiles, middle tiles
+        int mechunk, mfchunk;  // several-launch step: the same
+        int achunk;            // one-launch acoustic step
     };
     std::vector<Tiles> tuned;
     // time loops without host work between steps replay a captured graph of several steps
@@ -120,6 +122,7 @@ struct fwi3d_ctx {
     // elastic / VTI steps: the fused kernel (fwi3d_tune FWI3D_TUNE_FUSED, default on) and the y
     // chunks of its middle and side tiles (FWI3D_TUNE_FCHUNK, FWI3D_TUNE_ECHUNK; 0: by grid size)
     bool use_fused = true;
+    int form_probe = -1;  // step form forced while fwi3d_autotune times it (-1: by the rule)
     int fused_chunk = 0;
     int fused_echunk = 0;
     // launches of the multi-launch fused step on the second stream (FWI3D_TUNE_OVERLAP): 0

@@ -382,6 +382,7 @@ int shell_edge_count(const Geom& g) { return edge_count(6, g.nx, g.ny, g.nz); }
 // coefficients exceed the 32-bit byte offsets of the one-launch steps (a face of 3.7 M points
 // and more for VTI, 11 M for the others).
 int step_form(const fwi3d_ctx* c, bool fwd_snap, int physics, const Geom& g) {
+    if (c->form_probe >= 0) return c->form_probe;
     if (!c->use_fused) return STEP_FLUX;
     const ClosureSizes s = closure_sizes(physics == FWI3D_VTI, g);
     const bool fits = std::max(s.zc, std::max(s.xc, s.yc)) * sizeof(float4) < (1ULL << 32);
@@ -523,20 +524,21 @@ MultiPlan multi_plan(BShot& d, const Geom& g, int TX, int ychunk, int fchunk, in
 }
 
 // Tile shape for a physics and grid: the autotuned one if fwi3d_autotune measured this
-// grid on the context, else the context's settings (fwi3d_tune). `echunk`: y chunk of
-// the fused kernel's side tiles, `fchunk` of its middle tiles.
-void tiles_for(const fwi3d_ctx* c, int physics, const Geom& g, int& TX, int& ychunk, int& echunk, int& fchunk) {
-    TX = c->tune_tx;
-    ychunk = c->tune_ychunk;
-    echunk = c->fused_echunk;
-    fchunk = c->fused_chunk;
+// grid on the context, else the context's settings (fwi3d_tune).
+fwi3d_ctx::Tiles tiles_for(const fwi3d_ctx* c, int physics, const Geom& g) {
+    fwi3d_ctx::Tiles r{physics, g.nx, g.ny, g.nz, c->tune_tx, c->tune_ychunk, c->fused_echunk, c->fused_chunk,
+                       c->fused_echunk, c->fused_chunk, c->tune_ychunk};
     for (const auto& t : c->tuned)
         if (t.physics == physics && t.nx == g.nx && t.ny == g.ny && t.nz == g.nz) {
-            TX = t.tx;
-            ychunk = t.ychunk;
-            if (t.echunk > 0) echunk = t.echunk;
-            if (t.fchunk > 0) fchunk = t.fchunk;
+            r.tx = t.tx;
+            r.ychunk = t.ychunk;
+            if (t.echunk > 0) r.echunk = t.echunk;
+            if (t.fchunk > 0) r.fchunk = t.fchunk;
+            if (t.mechunk > 0) r.mechunk = t.mechunk;
+            if (t.mfchunk > 0) r.mfchunk = t.mfchunk;
+            if (t.achunk > 0) r.achunk = t.achunk;
         }
+    return r;
 }
 
 // ---- snapshot store: slot k holds forward step k*sub; unwritten slots read as zero.
@@ -729,14 +731,14 @@ void propagate_acoustic(fwi3d_ctx* c, bool adj, const float* d_model, const floa
     float* curr = F + n;
     float* next = F + 2 * n;
 
-    int TX, ychunk, echunk, fchunk;
-    tiles_for(c, FWI3D_ACOUSTIC, g, TX, ychunk, echunk, fchunk);
+    const fwi3d_ctx::Tiles tiles = tiles_for(c, FWI3D_ACOUSTIC, g);
+    const int TX = tiles.tx;
     AcuArgs A{};
     A.K = M; A.b = M + n; A.tz2 = tp.tz2; A.tx2 = tp.tx2; A.ty2 = tp.ty2; A.g = g;
     for (int f = 0; f < 6; f++) A.bc[f] = par->bc[f];
     A.dt = dt; A.dt2 = dt * dt;
     A.alpha = 0.2508560249f / par->free_surface_stiffness;
-    const int nblk = tile_grid_yc(A, g, TX, true, ychunk);
+    const int nblk = tile_grid_yc(A, g, TX, true, tiles.ychunk);
     const int nshell = shell_count(6, g.nx, g.ny, g.nz);  // points within 6 cells of a face
     // one-shot table for the time-step kernels (rotation from the step index)
     BShot T1h{};
@@ -755,7 +757,7 @@ void propagate_acoustic(fwi3d_ctx* c, bool adj, const float* d_model, const floa
     int nfused = 0;
     if (fused) {
         c->aux.ensure(aux);
-        nfused = acoustic_fused_plan(c->stream, T1h, d_src, c->aux.as<char>(), c->tune_ychunk);
+        nfused = acoustic_fused_plan(c->stream, T1h, d_src, c->aux.as<char>(), tiles.achunk);
     }
     const BShot* T1 = upload_shot1(c, T1h);
 
@@ -995,8 +997,8 @@ void propagate_elastic(fwi3d_ctx* c, bool vti, bool adj, const float* d_model, c
     };
     inject(prev, 0, 1);
 
-    int TX, ychunk, echunk, fchunk;
-    tiles_for(c, vti ? FWI3D_VTI : FWI3D_ELASTIC, g, TX, ychunk, echunk, fchunk);
+    const fwi3d_ctx::Tiles tiles = tiles_for(c, phys, g);
+    const int TX = tiles.tx, ychunk = tiles.ychunk;
     const int nblk = tile_grid_yc(A, g, TX, false, ychunk);
     EArgs AI = A;
     const int nint = tile_grid_yc(AI, g, TX, true, ychunk);
@@ -1008,9 +1010,9 @@ void propagate_elastic(fwi3d_ctx* c, bool vti, bool adj, const float* d_model, c
     T1h.nshell_blk = (T1h.nshell_pts + 255) / 256;
     const int nzslab = zslab_tiles(T1h.zs, g);
     MultiPlan MP{};
-    if (form == STEP_MULTI) MP = multi_plan(T1h, g, TX, ychunk, c->fused_chunk, c->fused_echunk);
+    if (form == STEP_MULTI) MP = multi_plan(T1h, g, TX, ychunk, tiles.mfchunk, tiles.mechunk);
     if (fused) {
-        fused_plan(T1h, g, fchunk, echunk);
+        fused_plan(T1h, g, tiles.fchunk, tiles.echunk);
         fused_tables(c->stream, vti, A, c->aux.as<float>(), T1h.ft);
     }
     T1h.I = I; T1h.src = d_src; T1h.ninj_blk = nbi;
@@ -1467,10 +1469,9 @@ int fwi3d_autotune(fwi3d_ctx* c, int physics, int nx, int ny, int nz, int steps,
     long long n0[fwi3d_ctx::kProfClasses];
     std::copy(c->prof_ms, c->prof_ms + fwi3d_ctx::kProfClasses, ms0);
     std::copy(c->prof_n, c->prof_n + fwi3d_ctx::kProfClasses, n0);
-    const bool uf0 = c->use_fused;
     const int tx0 = c->tune_tx, yc0 = c->tune_ychunk, ec0 = c->fused_echunk, fc0 = c->fused_chunk;
     auto restore = [&] {
-        c->use_fused = uf0; c->tune_tx = tx0; c->tune_ychunk = yc0; c->fused_echunk = ec0; c->fused_chunk = fc0;
+        c->form_probe = -1; c->tune_tx = tx0; c->tune_ychunk = yc0; c->fused_echunk = ec0; c->fused_chunk = fc0;
         c->prof = prof0; c->prof_steps_only = steps_only0;
         std::copy(ms0, ms0 + fwi3d_ctx::kProfClasses, c->prof_ms);
         std::copy(n0, n0 + fwi3d_ctx::kProfClasses, c->prof_n);
@@ -1481,6 +1482,8 @@ int fwi3d_autotune(fwi3d_ctx* c, int physics, int nx, int ny, int nz, int steps,
         REQUIRE(steps >= 1 && steps <= 1000, "steps must be 1..1000");
         HIP_OK(hipSetDevice(c->device));
         drain_events(c);
+        const Geom g = make_geom(nx, ny, nz, 1.f, 1.f, 1.f);
+        const bool acoustic = physics == FWI3D_ACOUSTIC;
         // a homogeneous synthetic model (vp 3, vs 1.7, rho 2.3, eps 0.1): the kernels'
         // timing does not depend on the values
         const size_t N = (size_t)nx * ny * nz;
@@ -1512,49 +1515,105 @@ int fwi3d_autotune(fwi3d_ctx* c, int physics, int nx, int ny, int nz, int steps,
                                           return t.physics == physics && t.nx == nx && t.ny == ny && t.nz == nz;
                                       }),
                        c->tuned.end());
-        auto run = [&](int tx, int yc) -> double {
+        // each form is timed with the parameters that its launches read, the better of two runs
+        // (10-step runs vary by a few per cent)
+        auto run = [&](int form, int tx, int yc) -> double {
+            c->form_probe = form;
             c->tune_tx = tx;
             c->tune_ychunk = yc;
             c->prof = true;
             c->prof_steps_only = true;
-            for (int k = 0; k < fwi3d_ctx::kProfClasses; k++) { c->prof_ms[k] = 0; c->prof_n[k] = 0; }
-            const int rc = fwi3d_propagate_device(c, physics, 0, m.as<float>(), m.as<float>(), nullptr, &none, &none,
-                                                  nullptr, &par, nx, ny, nz, 0.01f, 0.01f, 0.01f);
-            if (rc != FWI3D_OK) throw Err{rc, fwi3d::thread_error()};
-            return c->prof_ms[4] / steps;  // whole time steps (the kernels overlap)
+            double t = 1e30;
+            for (int rep = 0; rep < 2; rep++) {
+                for (int k = 0; k < fwi3d_ctx::kProfClasses; k++) { c->prof_ms[k] = 0; c->prof_n[k] = 0; }
+                const int rc = fwi3d_propagate_device(c, physics, 0, m.as<float>(), m.as<float>(), nullptr, &none, &none,
+                                                      nullptr, &par, nx, ny, nz, 0.01f, 0.01f, 0.01f);
+                if (rc != FWI3D_OK) throw Err{rc, fwi3d::thread_error()};
+                t = std::min(t, c->prof_ms[4] / steps);  // whole time steps (the kernels overlap)
+            }
+            return t;
         };
-        // the acoustic fused step has its rule; the tiles are those of the interior kernels
-        if (physics == FWI3D_ACOUSTIC) c->use_fused = false;
-        run(4, 8);  // warm-up
-        int best_tx = 4, best_yc = 8, best_ec = 0, best_fc = 0;
+        fwi3d_ctx::Tiles T{physics, nx, ny, nz, 4, 8, 0, 0, 0, 0, 0};
+        // the form of forward runs that fill a store (FWI3D_TUNE_FUSED 0: of every run): TX and the y
+        // chunk. The several-launch step reads the latter in its flux pass over the whole grid only,
+        // below 16 planes; elsewhere the default stays.
+        const int main_form = step_form(c, false, physics, g), base = acoustic || !c->use_fused ? STEP_FLUX : STEP_MULTI;
+        run(base, 4, 8);  // warm-up
         double best = 1e30;
         for (int tx : {4, 8})
             for (int yc : {4, 8, 16, 32}) {
-                const double t = run(tx, yc);
-                if (t < best) { best = t; best_tx = tx; best_yc = yc; }
+                if (base == STEP_MULTI && ny >= 16 && yc != T.ychunk) continue;
+                const double t = run(base, tx, yc);
+                if (t < best) { best = t; T.tx = tx; T.ychunk = yc; }
             }
-        if (physics != FWI3D_ACOUSTIC && c->use_fused && ny > 12) {
-            // y chunks of the fused kernel: the side tiles' and then the middle tiles' of the
-            // grid-size rule, scaled. Another chunk than the rule's must be 3 % faster: the
-            // timings of 10-step runs vary by a few per cent.
+        if (base == STEP_MULTI && ny > 12) {
+            // y chunk of its side tiles: about 0.6, 0.75, 1, 1.5, 2 or 2.5 side workgroups per CU
+            // (the edge tiles run one workgroup per CU; beside the middle tiles, fewer edge
+            // workgroups than CUs can be fastest: 256^3 414 against 451 us per step with 160 side
+            // workgroups). Another chunk than the grid-size rule's must be 3 % faster.
+            const int ntz = fused_tile_count(nz, FZ), ntx = fused_tile_count(nx, FW), nyo = ny - 12;
+            int tried[6], ntried = 0;
+            for (int target : {160, 192, 256, 384, 512, 640}) {
+                const int ec = fused_side_chunk(ntz, ntx, nyo, target);
+                if (std::find(tried, tried + ntried, ec) != tried + ntried) continue;
+                tried[ntried++] = ec;
+                c->fused_echunk = ec;
+                const double t = run(base, T.tx, T.ychunk);
+                if (t < 0.97 * best) { best = t; T.mechunk = ec; }
+            }
+            // middle tiles: one y chunk fewer or more per tile column than the rule's, unless the
+            // caller has set the chunk (the middle tiles share the CUs with the edge tiles)
+            c->fused_echunk = T.mechunk > 0 ? T.mechunk : ec0;
+            if (fc0 <= 0) {
+                const int mid = fused_middle_tiles(ntz, ntx);
+                const int want = std::max(1, 512 / std::max(1, mid > 0 ? mid : ntz * ntx));
+                const int rule = std::max(8, (nyo + want - 1) / want);
+                for (int w : {want - 1, want + 1}) {
+                    if (w < 1) continue;
+                    const int fc = std::max(8, (nyo + w - 1) / w);
+                    if (fc == rule) continue;
+                    c->fused_chunk = fc;
+                    const double t = run(base, T.tx, T.ychunk);
+                    if (t < 0.97 * best) { best = t; T.mfchunk = fc; }
+                }
+            }
+            c->fused_chunk = fc0;
+            c->fused_echunk = ec0;
+        }
+        if (acoustic && main_form == STEP_FUSED) {
+            // y chunk of the one-launch step: the rule's, scaled
+            const int rule = acoustic_tiles(g, 0).chunk;
+            T.achunk = rule;
+            best = run(STEP_FUSED, T.tx, rule);
+            for (int f : {2, 6, 8, 12}) {  // quarters
+                const int yc = std::max(1, f * rule / 4);
+                if (yc == rule) continue;
+                const double t = run(STEP_FUSED, T.tx, yc);
+                if (t < 0.97 * best) { best = t; T.achunk = yc; }
+            }
+        } else if (main_form == STEP_FUSED && ny > 12) {
+            // y chunks of the one-launch step: the side tiles' and then, unless the caller has set
+            // it, the middle tiles' of the rule, scaled
             BShot probe{};
-            fused_plan(probe, make_geom(nx, ny, nz, 1.f, 1.f, 1.f), fc0, ec0);
+            fused_plan(probe, g, fc0, ec0);
+            best = run(STEP_FUSED, T.tx, T.ychunk);
             for (double f : {0.6, 0.8, 1.25, 1.6}) {
                 c->fused_echunk = std::max(1, (int)(f * probe.ft.chunk[FC_SIDE]));
-                const double t = run(best_tx, best_yc);
-                if (t < 0.97 * best) { best = t; best_ec = c->fused_echunk; }
+                const double t = run(STEP_FUSED, T.tx, T.ychunk);
+                if (t < 0.97 * best) { best = t; T.echunk = c->fused_echunk; }
             }
-            c->fused_echunk = best_ec > 0 ? best_ec : ec0;
-            for (double f : {0.6, 0.8, 1.25, 1.6}) {
-                c->fused_chunk = std::max(1, (int)(f * probe.ft.chunk[FC_MID]));
-                const double t = run(best_tx, best_yc);
-                if (t < 0.97 * best) { best = t; best_fc = c->fused_chunk; }
-            }
+            c->fused_echunk = T.echunk > 0 ? T.echunk : ec0;
+            if (fc0 <= 0)
+                for (double f : {0.6, 0.8, 1.25, 1.6}) {
+                    c->fused_chunk = std::max(1, (int)(f * probe.ft.chunk[FC_MID]));
+                    const double t = run(STEP_FUSED, T.tx, T.ychunk);
+                    if (t < 0.97 * best) { best = t; T.fchunk = c->fused_chunk; }
+                }
         }
         restore();
-        c->tuned.push_back(fwi3d_ctx::Tiles{physics, nx, ny, nz, best_tx, best_yc, best_ec, best_fc});
-        if (tx_out) *tx_out = best_tx;
-        if (ychunk_out) *ychunk_out = best_yc;
+        c->tuned.push_back(T);
+        if (tx_out) *tx_out = T.tx;
+        if (ychunk_out) *ychunk_out = T.ychunk;
         m.release();
         return FWI3D_OK;
     } catch (const Err& e) {

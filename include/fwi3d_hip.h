@@ -162,13 +162,16 @@ enum fwi3d_tune_param {
 };
 int fwi3d_tune(fwi3d_ctx *ctx, int param, int value);
 /* Autotuner (no counterpart in the reference): times `steps` time steps of the given
- * physics and grid on a synthetic model for every tile shape (TX 4 or 8, y chunk 4, 8,
- * 16 or 32, and for the fused elastic / VTI step the y chunks of its side and of its middle
- * tiles, 0.6 to 1.6 times the grid-size rule's; another chunk than the rule's is kept when
- * it is at least 3 % faster) with HIP events, keeps the fastest for that
- * physics and grid on the context
- * (used by propagate and by batch admission in preference to fwi3d_tune's settings) and
- * returns it. */
+ * physics and grid on a synthetic model with HIP events, every step form that the context's
+ * runs take with the parameters that its launches read, and keeps the fastest for that physics
+ * and grid on the context (used by propagate and by batch admission in preference to
+ * fwi3d_tune's settings; chunks set by FWI3D_TUNE_FCHUNK are kept):
+ *   the form of forward runs with a snapshot store: TX 4 or 8 (*tx), y chunk 4, 8, 16 or 32
+ *     (*ychunk; 8 where no launch reads it), elastic / VTI: the y chunks of its side tiles (0.6
+ *     to 2.5 side workgroups per CU) and of its middle tiles;
+ *   the one-launch step: the y chunks of its side and of its middle tiles, 0.6 to 1.6 times
+ *     the grid-size rule's; acoustic: its y chunk, 0.5 to 3 times the rule's.
+ * Another chunk than the rule's is kept when it is at least 3 % faster. */
 int fwi3d_autotune(fwi3d_ctx *ctx, int physics, int nx, int ny, int nz, int steps, int *tx, int *ychunk);
 
 /* The snapshot store of the last forward call with sub > 0 on the context, decoded to

@@ -162,3 +162,16 @@ def test_y_chunks_reach_forward_runs_with_a_store():
     print(f"  us per step by the rule {us[0]:.0f}, one plane per chunk {us[1]:.0f}", flush=True)
     assert np.array_equal(out[0], out[1])
     assert us[1] > 1.5 * us[0]
+
+
+@pytest.mark.parametrize("physics", ["elastic", "vti"])
+def test_autotune_times_what_the_launches_read(physics):
+    """No launch of the elastic / VTI steps reads the y chunk of a grid of 16 planes or more: it
+    keeps the default, not the winner of equal timings."""
+    eng = F.Engine(0)
+    try:
+        picked = [eng.autotune(physics, (40 + 8 * k, 36, 50), steps=3) for k in range(4)]
+        print(f"  {picked}", flush=True)
+    finally:
+        eng.close()
+    assert all(tx in (4, 8) and yc == 8 for tx, yc in picked)
