@@ -308,7 +308,7 @@ def run_batch(args, torch, F, W, emit=True):
     resident = b.status()[1]
     torch.cuda.synchronize()
     t_admit = time.perf_counter() - t0
-    b.autotune(window=10)  # online: the first 40 steps time y chunks 4/8/16/32
+    b.autotune(window=10)  # online: with --unfused the first 40 steps time y chunks 4/8/16/32
     b.run()
     batch_tiles = b.tiles()
     torch.cuda.synchronize()
@@ -342,7 +342,7 @@ def run_batch(args, torch, F, W, emit=True):
         "batch_phase_s": {"admit": round(t_admit, 3), "steps": round(t_batch - t_admit, 3)},
         "autotuned_tiles_tx_ychunk": tiles,
         "batch_online_ychunk": batch_tiles[0],
-        "batch_candidate_ms_per_step": {str(y): round(t, 3) for y, t in zip((4, 8, 16, 32), batch_tiles[1])},
+        "batch_candidate_ms_per_step": {str(y): round(t, 3) for y, t in zip((4, 8, 16, 32), batch_tiles[1]) if t > 0},
         "traces_identical_to_plain": bool(same),
     }
     eng.close()

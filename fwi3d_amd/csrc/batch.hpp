@@ -139,6 +139,17 @@ void batch_rebuild(fwi3d_batch* b) {
     b->dirty = false;
 }
 
+// y chunk of the one-launch acoustic step for the batch's y chunk yc: the grid-size rule's at the
+// default 8, in proportion otherwise (the rule gives 1 to 6 planes, the interior kernels take 8).
+int batch_acoustic_chunk(const Geom& g, int yc) { return std::max(1, acoustic_tiles(g, 0).chunk * yc / 8); }
+
+// Whether a shot's launches read the batch's y chunk (the fused elastic / VTI steps have their own).
+bool batch_reads_ychunk(const fwi3d_batch* b) {
+    for (const auto& sh : b->shots)
+        if (sh.d.phys == FWI3D_ACOUSTIC || sh.d.form == STEP_FLUX) return true;
+    return false;
+}
+
 // Re-tile every shot of the batch with y chunk yc (block counts change, results do not).
 void batch_retile(fwi3d_batch* b, int yc) {
     using B = fwi3d_batch;
@@ -146,6 +157,7 @@ void batch_retile(fwi3d_batch* b, int yc) {
         BShot& d = sh.d;
         if (d.phys == FWI3D_ACOUSTIC) {
             if (d.form == STEP_FLUX) sh.nblk[B::C_AINT] = tile_grid_yc(d.a, d.g, b->TX, true, yc);
+            else sh.nblk[B::C_AFUSED] = acoustic_fused_tiles(d, batch_acoustic_chunk(d.g, yc));
         } else if (d.form == STEP_FLUX) {  // (the fused kernels keep their own y chunks)
             const bool e = d.phys == FWI3D_ELASTIC;
             sh.nblk[e ? B::C_EFLUX : B::C_VFLUX] = tile_grid_yc(d.ef, d.g, b->TX, false, yc);
@@ -483,7 +495,8 @@ int batch_add_impl(fwi3d_batch* b, int mode, int physics, const float* d_model, 
             A.prev = F; A.curr = F + n; A.next = F + 2 * n;
             if (step_form(c, mode == 1, physics, g) == STEP_FUSED) {
                 for (int k : {B::C_AINT, B::C_ASHELL, B::C_AINJ}) s.nblk[k] = 0;
-                s.nblk[B::C_AFUSED] = acoustic_fused_plan(st, d, d_src, (char*)aux, tiles.achunk);
+                s.nblk[B::C_AFUSED] = acoustic_fused_plan(
+                    st, d, d_src, (char*)aux, b->force_yc > 0 ? batch_acoustic_chunk(g, b->force_yc) : tiles.achunk);
             }
             if (d.I.ntgt > 0)
                 hipLaunchKernelGGL(acoustic_inject, dim3(d.ninj_blk), dim3(256), 0, st, F, A, d.I, d_src, d.nt, 0, 1);
@@ -562,6 +575,15 @@ int batch_add_impl(fwi3d_batch* b, int mode, int physics, const float* d_model, 
         if (smem) (void)hipFreeAsync(smem, c->stream);
         return fail(c, e);
     }
+}
+
+// End the online tuning: keep the fastest of the candidates timed so far.
+void batch_end_tuning(fwi3d_batch* b) {
+    int best = 0;
+    for (int k = 1; k < b->tune_idx; k++)
+        if (b->tune_ms[k] < b->tune_ms[best]) best = k;
+    batch_retile(b, b->tune_cands[best]);
+    b->tune_idx = -1;
 }
 
 // Drop the retired shots whose last work has completed: their events are destroyed and
@@ -645,8 +667,12 @@ int fwi3d_batch_step(fwi3d_batch* b, int nsteps, int* nactive) {
         b->last_retired.clear();
         batch_prune_retired(b);
         for (int q = 0; q < nsteps && !b->shots.empty(); q++) {
-            const bool tuning = b->tune_idx >= 0;
-            if (tuning && b->tune_left == b->tune_window) {  // a candidate's window starts
+            // a candidate's window starts only while a shot's launches read the y chunk: otherwise
+            // every candidate is the same work, and the steps keep their graph
+            const bool starts = b->tune_idx >= 0 && b->tune_left == b->tune_window;
+            const bool tuning = b->tune_idx >= 0 && (!starts || batch_reads_ychunk(b));
+            if (starts && !tuning && b->tune_idx > 0) batch_end_tuning(b);
+            if (starts && tuning) {
                 batch_retile(b, b->tune_cands[b->tune_idx]);
                 batch_rebuild(b);
                 HIP_OK(hipEventRecord(b->tev[0], c->stream));
@@ -726,11 +752,7 @@ int fwi3d_batch_step(fwi3d_batch* b, int nsteps, int* nactive) {
                 HIP_OK(hipEventElapsedTime(&ms, b->tev[0], b->tev[1]));
                 b->tune_ms[b->tune_idx] = ms / (b->tune_window - b->tune_left);
                 if (++b->tune_idx == fwi3d_batch::NCAND || b->shots.empty()) {
-                    int best = 0;
-                    for (int k = 1; k < b->tune_idx; k++)
-                        if (b->tune_ms[k] < b->tune_ms[best]) best = k;
-                    batch_retile(b, b->tune_cands[best]);
-                    b->tune_idx = -1;
+                    batch_end_tuning(b);
                 } else {
                     b->tune_left = b->tune_window;
                 }

@@ -669,6 +669,15 @@ size_t acoustic_aux_bytes(const Geom& g, const fwi3d_injector* inj) {
            ((size_t)g.ny * fused_tile_count(g.nx, FW) * fused_tile_count(g.nz, FZ) + 2 + nc + 2 * nc) * 4;
 }
 
+// Tile the step of shot d, whose source map is known (chunk: y planes per workgroup, 0 by grid
+// size). Returns the workgroups of its launch: the tiles, then those of the injection values.
+int acoustic_fused_tiles(BShot& d, int chunk) {
+    const AcuTabs tab = d.at.tab;
+    d.at = acoustic_tiles(d.g, chunk);
+    d.at.tab = tab;
+    return d.at.ntz * d.at.ntx * d.at.nyc + (d.im.nv + FTHREADS - 1) / FTHREADS;
+}
+
 // Plan the step of shot d and fill its tables, source map and first injection values in `base`
 // (acoustic_aux_bytes). Returns the workgroups of its launch.
 int acoustic_fused_plan(hipStream_t st, BShot& d, const float* src, char* base, int chunk) {
@@ -679,7 +688,6 @@ int acoustic_fused_plan(hipStream_t st, BShot& d, const float* src, char* base, 
     T.tab = acoustic_tabs((float4*)base, g);
     const long long nf = 2LL * ((long long)g.ny * g.nx + (long long)g.ny * g.nz + (long long)g.nx * g.nz);
     hipLaunchKernelGGL(acoustic_tables, dim3((unsigned)((nf + 255) / 256)), dim3(256), 0, st, d.a, T.tab);
-    int nblk = T.ntz * T.ntx * T.nyc;
     d.im = InjMap{};
     const InjTab& I = d.I;
     if (I.ntgt > 0) {
@@ -700,9 +708,8 @@ int acoustic_fused_plan(hipStream_t st, BShot& d, const float* src, char* base, 
         hipLaunchKernelGGL(inj_map_list, bt, th, 0, st, (const uint2*)mask, I, g, perm);
         const int nb = (d.im.nv + FTHREADS - 1) / FTHREADS;
         hipLaunchKernelGGL(acoustic_inj_first, dim3(nb), dim3(FTHREADS), 0, st, d.a, I, d.im, src, d.nt);
-        nblk += nb;
     }
-    return nblk;
+    return acoustic_fused_tiles(d, chunk);
 }
 
 void propagate_acoustic(fwi3d_ctx* c, bool adj, const float* d_model, const float* d_src, float* d_rcv,

@@ -351,8 +351,11 @@ int fwi3d_batch_wait(fwi3d_batch *b);
 int fwi3d_batch_status(const fwi3d_batch *b, int *nshots, long long *resident_bytes, int *step);
 /* Online tile tuning of the batch (no counterpart in the reference): the next 4 x window
  * steps run with y chunks 4, 8, 16 and 32 in turn (window steps each, timed with HIP
- * events), then the fastest is kept for every shot, present and future. Results do not
- * depend on the tiling. fwi3d_batch_tiles returns the y chunk in force (0: per shot)
+ * events), then the fastest is kept for every shot, present and future; the one-launch
+ * acoustic step takes the chunk in proportion, 8 being its grid-size rule's. A window waits
+ * for a shot whose launches read the chunk (the one-launch elastic / VTI step has chunks of
+ * its own); without any, no candidate is timed. Results do not depend on the tiling.
+ * fwi3d_batch_tiles returns the y chunk in force (0: per shot)
  * and, if cand_ms is not NULL, the measured milliseconds per step of the 4 candidates. */
 int fwi3d_batch_autotune(fwi3d_batch *b, int window);
 int fwi3d_batch_tiles(const fwi3d_batch *b, int *ychunk, float *cand_ms);

@@ -256,3 +256,39 @@ def test_batch_snapshot_store_errors_and_footprint():
         b.close()
     finally:
         eng.close()
+
+
+def test_online_tuning_waits_for_a_shot_that_reads_the_chunk():
+    """No launch of a one-launch elastic / VTI shot reads the batch's y chunk: a batch of these
+    times no candidate; the windows start when an acoustic shot joins, and the traces keep
+    their bits through the re-tilings."""
+    import torch
+    dev = torch.device("cuda:0")
+    shots = [make_shot("elastic", (30, 34, 38), 80, 2), make_shot("acoustic", (40, 44, 48), 70, 1)]
+    eng = F.Engine(0)
+    try:
+        b = F.Batch(eng)
+        b.autotune(3)
+        keep, out = [], []
+
+        def admit(s):
+            m, src = torch.from_numpy(s["model"]).to(dev), torch.from_numpy(s["src"]).to(dev)
+            r = torch.zeros((F.n_comp(F.PHYSICS[s["physics"]]), s["ext"].npts, s["par"].nt), device=dev)
+            torch.cuda.synchronize()
+            keep.extend([m, src])
+            out.append(r)
+            b.add(s["physics"], m.data_ptr(), src.data_ptr(), r.data_ptr(), s["inj"], s["ext"], s["par"], s["shape"],
+                  (H, H, H))
+
+        admit(shots[0])
+        b.step(20)
+        assert b.tiles() == (0, [0.0] * 4)
+        admit(shots[1])
+        b.run()
+        yc, ms = b.tiles()
+        assert yc in (4, 8, 16, 32) and all(t > 0 for t in ms)
+        b.close()
+        for s, r in zip(shots, out):
+            assert np.array_equal(r.cpu().numpy(), single(eng, s, dev)), s["physics"]
+    finally:
+        eng.close()
