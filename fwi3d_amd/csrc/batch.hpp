@@ -68,6 +68,7 @@ struct fwi3d_batch {
     std::vector<int> hmaps;
     std::vector<fwi3d::BShot> htab;
     size_t resident = 0;
+    bool lean = false;  // admit shots without the one-launch step's boundary data
     int force_yc = 0;  // y chunk of every shot (0: each shot's choice at admission)
     // online tile tuning: the candidate y chunks each run `tune_window` real steps of the
     // batch (results do not depend on the tiling), then the fastest is kept
@@ -89,16 +90,22 @@ using fwi3d::BShot;
 
 int batch_group(int phys) { return phys == FWI3D_ACOUSTIC ? 0 : (phys == FWI3D_ELASTIC ? 1 : 2); }
 
-// Device bytes of one batched shot: three wavefield sets, model, flux buffer, tapers,
-// injector tables (256-byte aligned parts).
-size_t batch_shot_bytes(int phys, const Geom& g, const fwi3d_injector* inj, const fwi3d_injector* ext) {
+// Bytes of a batched shot's flux buffer or boundary data (acoustic: tables and source map of the
+// one-launch step only).
+size_t batch_aux_bytes(int phys, const Geom& g, const fwi3d_injector* inj, int form) {
+    if (phys == FWI3D_ACOUSTIC) return form == STEP_FUSED ? acoustic_aux_bytes(g, inj) : 0;
+    return aux_bytes(phys == FWI3D_VTI, g, form);
+}
+
+// Device bytes of one batched shot that takes the step form `form`: three wavefield sets, model,
+// flux buffer or boundary data, tapers, injector tables (256-byte aligned parts).
+size_t batch_shot_bytes(int phys, const Geom& g, const fwi3d_injector* inj, const fwi3d_injector* ext, int form) {
     auto al = [](size_t x) { return (x + 255) / 256 * 256; };
     const int ncomp = phys == FWI3D_ACOUSTIC ? 1 : 3;
     const int nmf = phys == FWI3D_ACOUSTIC ? 2 : (phys == FWI3D_ELASTIC ? 3 : 7);
     const size_t n = (size_t)g.n;
-    const size_t aux = phys == FWI3D_ACOUSTIC ? acoustic_aux_bytes(g, inj) : aux_bytes(phys == FWI3D_VTI, g);
-    return al(3 * ncomp * n * 4) + al(nmf * n * 4) + al(aux) + al((size_t)(g.nz + g.nx + g.ny) * 4) +
-           al(inj_bytes(inj)) + al(inj_bytes(ext));
+    return al(3 * ncomp * n * 4) + al(nmf * n * 4) + al(batch_aux_bytes(phys, g, inj, form)) +
+           al((size_t)(g.nz + g.nx + g.ny) * 4) + al(inj_bytes(inj)) + al(inj_bytes(ext));
 }
 
 // Rebuild the device tables after shots joined or left.
@@ -358,13 +365,30 @@ long long fwi3d_batch_footprint(int physics, int nx, int ny, int nz, const fwi3d
     if (physics != FWI3D_ACOUSTIC && physics != FWI3D_ELASTIC && physics != FWI3D_VTI) return -1;
     try {
         const Geom g = make_geom(nx, ny, nz, 1.f, 1.f, 1.f);
-        return (long long)batch_shot_bytes(physics, g, inj, ext);
+        const fwi3d_ctx rule;  // the default settings' form of a shot without a store, which needs the most
+        return (long long)batch_shot_bytes(physics, g, inj, ext, step_form(&rule, false, physics, g));
     } catch (const Err&) {
         return -1;
     }
 }
 
 }  // extern "C"
+
+namespace fwi3d {
+
+long long batch_shot_need(const fwi3d_batch* b, int mode, bool lean, int physics, int nx, int ny, int nz,
+                          const fwi3d_injector* inj, const fwi3d_injector* ext) {
+    try {
+        const Geom g = make_geom(nx, ny, nz, 1.f, 1.f, 1.f);
+        const int form = step_form(b->c, mode == 1, physics, g);
+        return (long long)batch_shot_bytes(physics, g, inj, ext, form == STEP_FUSED && lean ? lean_form(physics) : form);
+    } catch (const Err&) {
+        return -1;
+    }
+}
+void batch_set_lean(fwi3d_batch* b, bool lean) { b->lean = lean; }
+
+}  // namespace fwi3d
 
 namespace {
 
@@ -409,9 +433,22 @@ int batch_add_impl(fwi3d_batch* b, int mode, int physics, const float* d_model, 
         HIP_OK(hipSetDevice(c->device));
         hipStream_t st = c->stream;
         const Geom g = make_geom(nx, ny, nz, dx, dy, dz);
-        const size_t bytes = batch_shot_bytes(physics, g, inj, ext);
-        if (hipMallocAsync(&mem, bytes, st) != hipSuccess || !mem)
-            throw Err{FWI3D_ENOMEM, "hipMallocAsync(" + std::to_string(bytes) + " bytes) for a batched shot failed"};
+        int form = step_form(c, mode == 1, physics, g);
+        if (form == STEP_FUSED && b->lean) form = lean_form(physics);
+        size_t bytes = batch_shot_bytes(physics, g, inj, ext, form);
+        auto get = [&] {
+            if (hipMallocAsync(&mem, bytes, st) == hipSuccess && mem) return true;
+            mem = nullptr;
+            (void)hipGetLastError();
+            return false;
+        };
+        bool got = get();
+        if (!got && form == STEP_FUSED && batch_shot_bytes(physics, g, inj, ext, lean_form(physics)) < bytes) {
+            form = lean_form(physics);
+            bytes = batch_shot_bytes(physics, g, inj, ext, form);
+            got = get();
+        }
+        if (!got) throw Err{FWI3D_ENOMEM, "hipMallocAsync(" + std::to_string(bytes) + " bytes) for a batched shot failed"};
         fwi3d_batch::Store store;
         if (mode == 1) {
             const int ncomp = physics == FWI3D_ACOUSTIC ? 1 : 3;
@@ -447,7 +484,7 @@ int batch_add_impl(fwi3d_batch* b, int mode, int physics, const float* d_model, 
         char* p = (char*)mem;
         float* F = (float*)p;          p += al(3 * ncomp * n * 4);
         float* M = (float*)p;          p += al(nmf * n * 4);
-        float* aux = (float*)p;        p += al(physics == FWI3D_ACOUSTIC ? acoustic_aux_bytes(g, inj) : aux_bytes(physics == FWI3D_VTI, g));
+        float* aux = (float*)p;        p += al(batch_aux_bytes(physics, g, inj, form));
         float* tp = (float*)p;         p += al((size_t)(g.nz + g.nx + g.ny) * 4);
         char* pinj = p;                p += al(inj_bytes(inj));
         char* pext = p;
@@ -493,7 +530,7 @@ int batch_add_impl(fwi3d_batch* b, int mode, int physics, const float* d_model, 
             s.nblk[B::C_ASHELL] = d.nshell_blk;
             s.nblk[B::C_AINJ] = d.ninj_blk;
             A.prev = F; A.curr = F + n; A.next = F + 2 * n;
-            if (step_form(c, mode == 1, physics, g) == STEP_FUSED) {
+            if (form == STEP_FUSED) {
                 for (int k : {B::C_AINT, B::C_ASHELL, B::C_AINJ}) s.nblk[k] = 0;
                 s.nblk[B::C_AFUSED] = acoustic_fused_plan(
                     st, d, d_src, (char*)aux, b->force_yc > 0 ? batch_acoustic_chunk(g, b->force_yc) : tiles.achunk);
@@ -522,7 +559,7 @@ int batch_add_impl(fwi3d_batch* b, int mode, int physics, const float* d_model, 
             d.nshell_blk = (d.nshell_pts + 255) / 256;
             s.nblk[grp == 1 ? B::C_ESHELL : B::C_VSHELL] = 0;  // the edges run in the slab class
             s.nblk[grp == 1 ? B::C_EZS : B::C_VZS] = zslab_tiles(d.zs, g) + 3 * d.nshell_blk;
-            d.form = step_form(c, mode == 1, physics, g);
+            d.form = form;
             if (d.form != STEP_FLUX)
                 for (int k : {B::C_EFLUX, B::C_VFLUX, B::C_EINT, B::C_VINT, B::C_EZS, B::C_VZS}) s.nblk[k] = 0;
             // the single-shot path's plan with the context's fused y chunks, not the autotuned

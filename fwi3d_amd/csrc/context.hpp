@@ -35,17 +35,27 @@ struct DevBuf {
     void* p = nullptr;
     size_t bytes = 0;
     bool borrowed = false;
-    void ensure(size_t nb) {
-        if (nb <= bytes) return;
-        if (borrowed)
-            throw Err{FWI3D_ENOMEM, "workspace slice of " + std::to_string(bytes) + " bytes is too small for " +
-                                        std::to_string(nb) + " bytes"};
+    // Hold at least nb bytes; false if the memory cannot be had (the buffer may then be empty).
+    bool grow(size_t nb) {
+        if (nb <= bytes) return true;
+        if (borrowed) return false;
         if (p) (void)hipFree(p);
         p = nullptr;
         bytes = 0;
-        hipError_t e = hipMalloc(&p, nb);
-        if (e != hipSuccess) throw Err{FWI3D_ENOMEM, "hipMalloc(" + std::to_string(nb) + " bytes) failed"};
+        if (hipMalloc(&p, nb) != hipSuccess) {
+            p = nullptr;
+            (void)hipGetLastError();  // (the failure is reported here, not by the next call)
+            return false;
+        }
         bytes = nb;
+        return true;
+    }
+    void ensure(size_t nb) {
+        if (grow(nb)) return;
+        if (borrowed)
+            throw Err{FWI3D_ENOMEM, "workspace slice of " + std::to_string(bytes) + " bytes is too small for " +
+                                        std::to_string(nb) + " bytes"};
+        throw Err{FWI3D_ENOMEM, "hipMalloc(" + std::to_string(nb) + " bytes) failed"};
     }
     void release() {
         if (p && !borrowed) (void)hipFree(p);
@@ -145,6 +155,14 @@ struct fwi3d_ctx {
 };
 
 namespace fwi3d {
+
+// Device bytes of a shot of the batch (mode 0 forward, 1 forward with a snapshot store, 2
+// adjoint; without the store itself), -1 for a grid it cannot take. lean: in the step form that
+// needs no boundary coefficients.
+long long batch_shot_need(const fwi3d_batch* b, int mode, bool lean, int physics, int nx, int ny, int nz,
+                          const fwi3d_injector* inj, const fwi3d_injector* ext);
+// Shots admitted from here on take that form (or again the rule's).
+void batch_set_lean(fwi3d_batch* b, bool lean);
 
 inline void set_error(fwi3d_ctx* c, const std::string& msg) {
     thread_error() = msg;

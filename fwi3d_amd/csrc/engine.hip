@@ -389,11 +389,16 @@ int step_form(const fwi3d_ctx* c, bool fwd_snap, int physics, const Geom& g) {
     return fwd_snap || !fits ? STEP_MULTI : STEP_FUSED;
 }
 
-// Bytes of the flux buffer of a shot, which the fused step uses for its boundary tables and
+// Form of a shot that cannot have the memory of the one-launch step's boundary data.
+int lean_form(int physics) { return physics == FWI3D_ACOUSTIC ? STEP_FLUX : STEP_MULTI; }
+
+// Bytes of the flux buffer of a shot, which the one-launch step uses for its boundary tables and
 // dt^2 / rho instead (more than the fluxes on grids a few tens of points wide).
 size_t flux_bytes(bool vti, const Geom& g) { return (size_t)(vti ? 9 : 7) * g.n * sizeof(float); }
 size_t fused_bytes(bool vti, const Geom& g) { return closure_sizes(vti, g).total() * sizeof(float4) + (size_t)g.n * sizeof(float); }
-size_t aux_bytes(bool vti, const Geom& g) { return std::max(flux_bytes(vti, g), fused_bytes(vti, g)); }
+size_t aux_bytes(bool vti, const Geom& g, int form) {
+    return form == STEP_FUSED ? std::max(flux_bytes(vti, g), fused_bytes(vti, g)) : flux_bytes(vti, g);
+}
 
 // Fill the boundary data of the fused step in `base` (fused_bytes).
 void fused_tables(hipStream_t st, bool vti, const EArgs& A, float* base, FusedTiles& F) {
@@ -758,12 +763,11 @@ void propagate_acoustic(fwi3d_ctx* c, bool adj, const float* d_model, const floa
     T1h.E = E; T1h.rcv = d_rcv; T1h.next_blk = (E.npts + 127) / 128;
     // A forward run that fills a snapshot store keeps the interior / shell kernels, whose
     // rounding the codes of 16-bit stores have (the traces do not depend on the store's format).
-    // So does a shot that fits a fixed workspace only without the tables.
+    // So does a shot that fits the fixed workspace or the card only without the tables.
     const size_t aux = acoustic_aux_bytes(g, inj);
-    const bool fused = step_form(c, fwd_snap, FWI3D_ACOUSTIC, g) == STEP_FUSED && !(c->aux.borrowed && c->aux.bytes < aux);
+    const bool fused = step_form(c, fwd_snap, FWI3D_ACOUSTIC, g) == STEP_FUSED && c->aux.grow(aux);
     int nfused = 0;
     if (fused) {
-        c->aux.ensure(aux);
         nfused = acoustic_fused_plan(c->stream, T1h, d_src, c->aux.as<char>(), tiles.achunk);
     }
     const BShot* T1 = upload_shot1(c, T1h);
@@ -955,13 +959,13 @@ void propagate_elastic(fwi3d_ctx* c, bool vti, bool adj, const float* d_model, c
     const int nmf = vti ? 7 : 3;  // device model fields (VTI adds c11b)
     c->fields.ensure(9 * n * sizeof(float));
     c->model.ensure(nmf * n * sizeof(float));
-    // the flux buffer, T (1 or 3) and 6 shear fluxes; or the one-launch step's boundary data. (A
-    // fixed workspace that holds the fluxes but not that data, on a narrow grid, runs the
-    // several-launch step, which needs only the fluxes of the y faces.)
+    // the flux buffer, T (1 or 3) and 6 shear fluxes; or the one-launch step's boundary data. (Where
+    // the fixed workspace or the card holds the fluxes but not that data, on a narrow grid, the
+    // several-launch step runs, which needs only the fluxes of the y faces.)
     int form = step_form(c, !adj && par->sub > 0, vti ? FWI3D_VTI : FWI3D_ELASTIC, g);
-    if (form == STEP_FUSED && c->aux.borrowed && c->aux.bytes < fused_bytes(vti, g)) form = STEP_MULTI;
+    if (form == STEP_FUSED && !c->aux.grow(aux_bytes(vti, g, form))) form = lean_form(vti ? FWI3D_VTI : FWI3D_ELASTIC);
     const bool fused = form == STEP_FUSED;
-    c->aux.ensure(fused ? aux_bytes(vti, g) : flux_bytes(vti, g));
+    c->aux.ensure(aux_bytes(vti, g, form));
     float* F = c->fields.as<float>();
     float* Mf = c->model.as<float>();
     HIP_OK(hipMemsetAsync(F, 0, 9 * n * sizeof(float), c->stream));
@@ -1346,7 +1350,7 @@ int fwi3d_propagate_device_noalloc(fwi3d_ctx* c, int physics, int adj, const flo
         for (size_t x : sz) total += x;
         // (the fused step's boundary data where it needs more than the fluxes and still fits)
         if (c->use_fused && total <= kScratchBytes) {
-            const size_t more = al(ac ? acoustic_aux_bytes(g, inj) : aux_bytes(physics == FWI3D_VTI, g)) - sz[2];
+            const size_t more = al(ac ? acoustic_aux_bytes(g, inj) : aux_bytes(physics == FWI3D_VTI, g, STEP_FUSED)) - sz[2];
             if (total + more <= kScratchBytes) {
                 sz[2] += more;
                 total += more;

@@ -17,6 +17,8 @@
 // and the preparation of new requests overlaps the batch's kernels on the side stream.
 // Each request computes exactly what fwi3d_apply_forward_device /
 // fwi3d_fwi_shot_device compute for it alone (same kernels, same order of operations).
+// (A request that the whole budget holds only without the one-launch step's boundary data
+// takes the other step form, and agrees with them to rounding.)
 //
 // Included once, by operator.hip (it uses that file's kernels and host helpers).
 #pragma once
@@ -46,6 +48,7 @@ struct fwi3d_server {
         float *conv = nullptr, *srcp = nullptr, *rcvp = nullptr, *tmp = nullptr, *syn = nullptr;
         unsigned* red = nullptr;
         double *g64 = nullptr, *dmis = nullptr;
+        bool lean = false;  // its shots take the step form without boundary data
         int shot = -1;  // current shot id in the batch
         hipEvent_t done = nullptr;
         double t_submit = 0, t_admit = 0, t_done = 0;
@@ -115,12 +118,16 @@ size_t req_rest_bytes(const SReq& q) {
     return b;
 }
 
-// Device bytes the request's shots hold in the batch (one shot at a time; a gradient
-// request adds its snapshot store).
-size_t req_batch_bytes(const SReq& q) {
-    long long b = fwi3d_batch_footprint(q.d.physics, q.d.nx, q.d.ny, q.d.nz, &q.si.t, &q.ri.t);
-    REQUIRE(b > 0, "request grid not admissible to a batch");
-    if (q.r.kind == FWI3D_REQ_GRADIENT) {
+// Device bytes the request's shots hold in the batch (one shot at a time, forward and adjoint;
+// a gradient request adds its snapshot store). lean: batch_shot_need.
+size_t req_batch_bytes(const Srv* s, const SReq& q, bool lean) {
+    const bool grad = q.r.kind == FWI3D_REQ_GRADIENT;
+    const fwi3d_injector none{};
+    REQUIRE(fwi3d_batch_footprint(q.d.physics, q.d.nx, q.d.ny, q.d.nz, &q.si.t, &q.ri.t) > 0,
+            "request grid not admissible to a batch");
+    long long b = batch_shot_need(s->b, grad ? 1 : 0, lean, q.d.physics, q.d.nx, q.d.ny, q.d.nz, &q.si.t, &q.ri.t);
+    if (grad) {
+        b = std::max(b, batch_shot_need(s->b, 2, lean, q.d.physics, q.d.nx, q.d.ny, q.d.nz, &q.ri.t, &none));
         const long long sb = fwi3d_batch_snap_footprint(q.d.physics, q.d.nx, q.d.ny, q.d.nz, q.par.nt, q.par.sub,
                                                         q.par.snap_precision);
         REQUIRE(sb > 0, "invalid snapshot store");
@@ -199,6 +206,7 @@ void srv_start(Srv* s, SReq* q) {
     HIP_OK(hipEventRecord(s->prep_ev, ps));
     HIP_OK(hipStreamWaitEvent(s->c->stream, s->prep_ev, 0));
     int id = -1;
+    batch_set_lean(s->b, q->lean);
     const int rc = fwi3d_batch_add(s->b, q->d.physics, q->conv, q->srcp, q->rcvp, &q->si.t, &q->ri.t, &q->pp, sh->nx,
                                    sh->ny, sh->nz, sh->dx, sh->dy, sh->dz, &id);
     if (rc != FWI3D_OK) throw Err{rc, fwi3d::thread_error()};
@@ -251,6 +259,7 @@ void srv_after_forward(Srv* s, SReq* q) {
     }
     HIP_OK(hipGetLastError());
     int id = -1;
+    batch_set_lean(s->b, q->lean);
     const int rc = fwi3d_batch_add_adjoint(s->b, q->shot, q->d.physics, q->conv, asrc, &q->ri.t, q->g64, &q->pp,
                                            sh->nx, sh->ny, sh->nz, sh->dx, sh->dy, sh->dz, &id);
     if (rc != FWI3D_OK) throw Err{rc, fwi3d::thread_error()};
@@ -332,7 +341,11 @@ void srv_admit(Srv* s) {
                 }
                 srv_analyse(s, q);
             }
-            const long long rest = (long long)(req_rest_bytes(*q) + req_batch_bytes(*q));
+            // a request that the whole budget holds only without the one-launch step's boundary
+            // data takes the step form that needs none
+            long long rest = (long long)(req_rest_bytes(*q) + req_batch_bytes(s, *q, false));
+            q->lean = (long long)q->reserved + rest > s->budget;
+            if (q->lean) rest = (long long)(req_rest_bytes(*q) + req_batch_bytes(s, *q, true));
             {
                 std::lock_guard<std::mutex> lk(s->mu);
                 in_use = s->in_use;

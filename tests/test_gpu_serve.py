@@ -170,3 +170,39 @@ def test_serve_budget_admission_and_errors():
     finally:
         srv.close()
         eng.close()
+
+
+@pytest.mark.parametrize("kind", ["model", "gradient"])
+def test_budget_without_room_for_boundary_tables(kind):
+    """A server whose budget holds an acoustic request but not the boundary coefficients of the
+    one-launch step serves it all the same, by the other step form (results to rounding)."""
+    import torch
+    dev = torch.device("cuda:0")
+    shape = (36, 30, 70)
+    ny, nx, nz = shape
+    over = dict(dt=0.0008, sub=4) if kind == "gradient" else dict(dt=0.0008)
+    eng = F.Engine(0)
+    try:
+        want = None
+        budget = 8 << 30
+        for turn in range(2):
+            q = build_request(3, kind, "acoustic", shape, 130, 0.0008, over, dev)
+            torch.cuda.synchronize()
+            srv = F.Server(eng, hbm_budget=budget, max_active=4)
+            rid = submit(srv, q)
+            srv.wait()
+            st = srv.stats()
+            assert srv.poll(rid)[0] == 2, srv.error(rid)
+            srv.close()
+            got = [q["data"].cpu().numpy()] + ([q["grad"].cpu().numpy()] if kind == "gradient" else [])
+            if turn == 0:
+                want, peak = got, st["hbm_peak"]
+                # (384 B of coefficients and 16 of face values per point of a face of each axis)
+                budget = peak - 400 * (ny * nx + ny * nz + nx * nz)
+        assert st["hbm_peak"] <= budget < peak
+        for g, w in zip(got, want):
+            e = float(np.linalg.norm(g - w) / np.linalg.norm(w))
+            print(f"  {kind}: rel L2 between the step forms {e:.1e}", flush=True)
+            assert np.abs(w).max() > 0 and e <= 1e-5  # rounding of a few hundred steps
+    finally:
+        eng.close()

@@ -45,6 +45,17 @@ def test_batch_shot_footprint_covers_fields_model_and_fluxes():
     assert F.Batch.footprint("vti", shape, inj, ext) > F.Batch.footprint("elastic", shape, inj, ext)
 
 
+def test_wide_face_footprint_holds_no_boundary_tables():
+    """A VTI shot whose boundary coefficients pass 4 GiB never takes the step that reads them:
+    its footprint is fields, model, fluxes and small tables."""
+    shape = (12, 1920, 1984)
+    cells = shape[0] * shape[1] * padded(shape[2])
+    d = (0.01, 0.01, 0.01)
+    inj, ext = F.Injector(1, [[0.5, 0.05, 0.5]], shape, d), F.Injector(0, [[0.6, 0.05, 0.5]], shape, d)
+    need = (3 * 3 + 7 + 9) * cells * 4
+    assert need <= F.Batch.footprint("vti", shape, inj, ext) <= need + (1 << 20)
+
+
 def test_serve_mix_is_seeded_and_follows_the_stream_spec():
     a, b = W.serve_mix(500, seed=42), W.serve_mix(500, seed=42)
     assert a == b and W.serve_mix(500, seed=43) != a
