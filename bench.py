@@ -87,13 +87,13 @@ ENGINE_TUNE = {}
 
 # profiled kernel classes of the elastic time step (fwi3d_profile_read), by step form
 KERNEL_CLASSES = {
-    True: ((0, "elastic_fused"),),
+    True: ((0, "elastic_fused"), (5, "elastic_multi_tiles"), (1, "elastic_multi_yflux"), (3, "elastic_multi_yslabs")),
     False: ((0, "elastic_interior"), (1, "elastic_flux"), (2, "elastic_boundary"), (3, "elastic_zslab")),
 }
 STEP_KERNEL = {
-    True: "elastic time step = one elastic_fused_step launch (all tiles and the receivers); in the forward run, which "
-          "fills the snapshot store, the fused middle and edge tiles, the y faces' flux pass and slabs on two streams "
-          "(HIP events around each step on the engine stream; traffic: the one-launch step's)",
+    True: "elastic time step, mean of both runs: adjoint one elastic_fused_step launch (all tiles and the receivers); "
+          "forward, which fills the snapshot store, elastic_multi tiles (middle and edge), the y faces' flux pass and "
+          "slabs on two streams (HIP events around each step on the engine stream; per-kernel averages on one stream)",
     False: "elastic time step = elastic_flux + elastic_interior + elastic_boundary + elastic_zslab launches "
            "(HIP events around each step on the engine stream)",
 }
@@ -115,12 +115,19 @@ def traffic_profile(n):
 
 def kernel_rooflines(fused, nz, nx, ny, avg_us, n):
     """Per kernel class of the elastic step: the cells it handles, its algorithmic bytes
-    (48 B per cell it updates: u, prev, lambda, mu, rho read, next written), its launch
-    time, achieved GB/s and fraction of 8 TB/s, and its measured HBM bytes per launch from the committed PMC summary when there is one."""
+    (48 B per cell it updates: u, prev, lambda, mu, rho read, next written; the y-face
+    flux pass reads u, lambda, mu and writes T and 6 fluxes, 48 B per cell too), its
+    one-stream launch time, achieved GB/s and fraction of 8 TB/s, and its measured HBM
+    bytes per launch from the committed PMC summary when there is one."""
     nxz = nx * nz
     if fused:
-        cells = {"elastic_fused": nxz * ny}
-        prof_keys = {"elastic_fused": ("elastic_fused_step",)}
+        # the one-launch step (adjoint); the several-launch step (forward with a store): tiles of the
+        # planes 6 cells inside the y faces, flux pass of the 8 and update of the 6 planes at each
+        cells = {"elastic_fused": nxz * ny, "elastic_multi_tiles": nxz * max(0, ny - 12),
+                 "elastic_multi_yflux": nxz * min(ny, 16), "elastic_multi_yslabs": nxz * min(ny, 12)}
+        prof_keys = {"elastic_fused": ("elastic_fused_step",),
+                     "elastic_multi_tiles": ("elastic_multi (middle tiles)", "elastic_multi (edge tiles)"),
+                     "elastic_multi_yflux": ("elastic_flux_batch (y faces)",), "elastic_multi_yslabs": ("elastic_yslabs_ext",)}
     else:
         inner = max(0, nx - 12) * max(0, ny - 12) * max(0, nz - 12)
         cells = {"elastic_interior": inner, "elastic_flux": nxz * ny, "elastic_boundary": 0,
@@ -375,8 +382,8 @@ def run_acoustic(args, torch, F, W):
     eng.tune(graphs=False)
     eng.profile(True)
     F.apply_forward_device(eng, par(), geo, False, model.data_ptr(), src.data_ptr(), data.data_ptr())
-    kern = {name: eng.profile_read(k) for k, name in ((0, "acoustic_interior"), (2, "acoustic_boundary"),
-                                                      (4, "acoustic_time_step_eager"))}
+    names = ((0, "acoustic_interior"), (2, "acoustic_boundary")) if args.unfused else ((0, "acoustic_fused_step"),)
+    kern = {name: eng.profile_read(k) for k, name in names + ((4, "acoustic_time_step_eager"),)}
     eng.profile(False)
     eng.tune(graphs=True)
     for _ in range(args.warmup):
@@ -418,7 +425,9 @@ def run_acoustic(args, torch, F, W):
         "trace_max_abs": float(data.abs().max()),
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": None,
-                     "kernel": "acoustic time step = acoustic_interior + acoustic_boundary (+ extraction, injection) "
+                     "kernel": ("acoustic time step = acoustic_interior + acoustic_boundary (+ extraction, injection) "
+                                if args.unfused else "acoustic time step = acoustic_fused_step (tiles, injection and "
+                                "receivers in one launch) ") +
                                "replayed from a captured graph (HIP events around each 16-step replay)",
                      "step_us": round(t_step * 1e6, 2), "bytes_per_cell": ACOUSTIC_BYTES_PER_CELL,
                      "cells_per_step": N, "avg_us": {k: round(v, 2) for k, v in avg_us.items()},

@@ -363,9 +363,9 @@ class Engine:
         self._check(lib().fwi3d_profile(self._h, level), "fwi3d_profile")
 
     def profile_read(self, kernel=0):
-        """(milliseconds, launches) of kernel class 0 (interior or fused time step), 1 (flux
-        pre-pass, elastic/VTI), 2 (boundary-shell time step) or 3 (z-slab time step,
-        elastic/VTI)."""
+        """(milliseconds, launches) of kernel class 0 (interior or one-launch time step), 1
+        (flux pre-pass, elastic/VTI), 2 (boundary-shell time step), 3 (z-slab time step,
+        elastic/VTI), 4 (whole time step) or 5 (fused tiles of the several-launch step)."""
         ms = C.c_double()
         n = C.c_longlong()
         self._check(lib().fwi3d_profile_read(self._h, int(kernel), C.byref(ms), C.byref(n)), "fwi3d_profile_read")

@@ -111,9 +111,6 @@ struct fwi3d_ctx {
     long long snap_n = 0;
     bool snap_valid = false;
     int snap_dims[3] = {0, 0, 0};
-    // profiling: [0] interior time-step kernel, [1] flux pre-pass (elastic/VTI),
-    // [2] boundary-shell time-step kernel, [3] slab kernel (elastic/VTI), [4] the whole
-    // time step (its kernels, launched one after another)
     // tiling of the y-marching kernels (fwi3d_tune)
     int tune_ychunk = 0;  // y planes per workgroup (0: default 8)
     int tune_tx = 4;      // x rows per workgroup (4 or 8)
@@ -142,9 +139,12 @@ struct fwi3d_ctx {
     fwi3d::DevBuf stepctr;
     std::vector<hipGraphExec_t> graph_execs;  // instantiated in the current call, freed after it
     std::vector<hipGraph_t> graphs;
+    // profiling: [0] interior time-step kernel or one-launch step, [1] flux pre-pass (elastic/VTI),
+    // [2] boundary-shell time-step kernel, [3] slab kernel (elastic/VTI), [4] the whole time step,
+    // [5] the several-launch step's fused tiles (the planes 6 cells inside the y faces)
     bool prof = false;
     bool prof_steps_only = false;  // record only whole-step events (fwi3d_profile level 2)
-    static constexpr int kProfClasses = 5;  // interior, flux, shell, z slabs, whole time step
+    static constexpr int kProfClasses = 6;
     double prof_ms[kProfClasses] = {};
     long long prof_n[kProfClasses] = {};
     std::vector<hipEvent_t> ev;

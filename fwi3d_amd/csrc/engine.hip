@@ -878,9 +878,9 @@ void step_elastic_multi(fwi3d_ctx* c, const BShot* T, StepIdx it, const MultiPla
     };
     const bool per_kernel = c->prof && !c->prof_steps_only;
     if (c->fused_overlap == 0 || per_kernel) {
-        // one stream (and per-kernel timing: classes 0 fused tiles, 1 flux pass, 3 slabs)
+        // one stream (and per-kernel timing: classes 5 fused tiles, 1 flux pass, 3 slabs)
         if (P.nfused + P.nfedge > 0)
-            timed(c, 0, [&] {
+            timed(c, 5, [&] {
                 middle(c->stream);
                 edge(c->stream);
             });

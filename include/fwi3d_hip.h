@@ -128,10 +128,12 @@ int fwi3d_propagate_device_noalloc(fwi3d_ctx *ctx, int physics, int adj, const f
  * resets), enable=2 only whole time steps (class 4: fewer event records in the timed
  * work), 0 stops.
  * read() returns the summed milliseconds and launch count since the last enable of
- * kernel class `kernel`: 0 = the interior time-step kernel (or the fused one), 1 = the elastic/VTI flux
- * pre-pass, 2 = the boundary-shell time-step kernel (elastic/VTI: the shell's edges and
+ * kernel class `kernel`: 0 = the interior time-step kernel or the one-launch step, 1 = the
+ * elastic/VTI flux pre-pass, 2 = the boundary-shell time-step kernel (elastic/VTI: the shell's edges and
  * corners), 3 = the elastic/VTI slab kernel (the z slabs away from the x and y faces and
- * the x and y slabs away from the other faces), 4 = the whole time step. */
+ * the x and y slabs away from the other faces), 4 = the whole time step, 5 = the fused tiles
+ * of the several-launch elastic/VTI step (middle and edge tiles, the planes 6 cells inside
+ * the y faces; its y faces are classes 1 and 3). */
 /* Tiling of the y-marching time-step kernels, per context (no counterpart in the
  * reference; the tile shapes an autotuner picks): FWI3D_TUNE_YCHUNK = y planes per
  * workgroup (0: default 8; the one-launch acoustic step: by grid size), FWI3D_TUNE_TX = x

@@ -334,3 +334,24 @@ def test_two_stream_step_is_launched_directly(eng):
     finally:
         eng.profile(False)
     assert n == nt - 1
+
+
+@pytest.mark.parametrize("physics", ["elastic", "vti"])
+def test_profile_classes_of_the_two_step_forms(eng, physics):
+    """Class 0 is the one-launch step; a forward run with a store counts its fused tiles as class
+    5 and its y faces as classes 1 and 3."""
+    shape, nt = (30, 34, 38), 21
+    model, src, sloc, rloc, d, dt = small_shot(physics, 1, shape=shape, nt=nt)
+    inj, ext = F.Injector(1, sloc, shape, d), F.Injector(0, rloc, shape, d)
+    got = {}
+    try:
+        for sub in (0, 4):
+            eng.tune(graphs=False)
+            eng.profile(True)
+            eng.propagate(physics, model, src, inj, ext, F.make_param(nt, dt, sub=sub), d)
+            got[sub] = [eng.profile_read(k)[1] for k in (0, 1, 2, 3, 5)]
+    finally:
+        eng.profile(False)
+        eng.tune(graphs=True)
+    assert got[0] == [nt - 1, 0, 0, 0, 0]
+    assert got[4] == [0, nt - 1, 0, nt - 1, nt - 1]
