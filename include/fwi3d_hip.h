@@ -94,7 +94,10 @@ int fwi3d_dipole_tables(const float *loc5, int npts, float gl, int nx, int ny, i
  *   grad   NULL (forward) or [ng][ny][nx][nz] accumulated (+=) imaging condition of
  *          compute_gradients (acoustic {K, 1/rho}: ng=2; elastic/VTI {lambda,mu,rho}: ng=3)
  * A forward call with par->sub > 0 stores the snapshots in the context; an adjoint
- * call reads the ones of the last forward call on the same context. */
+ * call reads the ones of the last forward call on the same context. Runs that fill a
+ * snapshot store take another step form than runs without one (fwi3d_tune): the traces of
+ * a shot agree to rounding between sub = 0 and sub > 0, bit for bit with FWI3D_TUNE_FUSED 0
+ * only. They do not depend on the value of sub > 0 or on the store's format. */
 int fwi3d_propagate(fwi3d_ctx *ctx, int physics, int adj, const float *model, const float *src, float *rcv,
                     const fwi3d_injector *inj, const fwi3d_injector *ext, float *grad, const fwi3d_param *par,
                     int nx, int ny, int nz, float dx, float dy, float dz);
