@@ -337,8 +337,9 @@ class Engine:
             self._check(lib().fwi3d_tune(self._h, 2, int(bool(graphs))), "fwi3d_tune")
 
     def autotune(self, physics, shape, steps=10):
-        """Measure every tile shape on this grid (fwi3d_autotune); the fastest is used for
-        this physics and grid from now on. Returns (tx, ychunk)."""
+        """Time the tilings of each step form on this grid (fwi3d_autotune); the fastest are
+        used for this physics and grid from now on. Returns (tx, ychunk) of the form of
+        forward runs with a snapshot store (ychunk 8 where no launch reads it)."""
         ph = PHYSICS[physics] if isinstance(physics, str) else int(physics)
         ny, nx, nz = shape
         tx, yc = C.c_int(), C.c_int()
@@ -472,7 +473,8 @@ class Batch:
         self.engine._check(lib().fwi3d_batch_wait(self._h), "fwi3d_batch_wait")
 
     def autotune(self, window=10):
-        """Time y chunks 4, 8, 16, 32 over the next 4 x window steps, then keep the best."""
+        """Time y chunks 4, 8, 16, 32 over the next 4 x window steps (once a shot's launches
+        read the chunk), then keep the best (fwi3d_batch_autotune)."""
         self.engine._check(lib().fwi3d_batch_autotune(self._h, int(window)), "fwi3d_batch_autotune")
 
     def tiles(self):

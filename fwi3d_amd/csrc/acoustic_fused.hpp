@@ -13,10 +13,10 @@
 //
 // Small grids are bound by the latency of a plane (load, barrier, update) times the planes of
 // a chunk, so the chunk is as short as fills the chip; large ones by HBM (20 B per cell).
-// Per step with its injection: (ny, nx, nz) = (40, 52, 47) 8.5 us, 100^3 17, 128^3 22, (203, 187,
-// 211) 56 (2.9 TB/s of the 20 B; 79 VGPRs, three workgroups per CU; the issue slots are about
-// half used), against 14, 21, 30 and 67 us with interior tiles, a point-wise shell and an
-// injection launch.
+// Per step with its injection (HIP events around graph replays): (ny, nx, nz) = (40, 52, 47) 6.7 us,
+// 100^3 16.6, 128^3 20, (203, 187, 211) 53.5 (3.0 TB/s of the 20 B; 79 VGPRs, three workgroups per
+// CU; the issue slots are about half used), against 13, 21.6, 29 and 65 us with interior tiles, a
+// point-wise shell and an injection launch.
 //
 // Injection. A word of mask and one of rank per 32 points mark the points that sources touch
 // (0.25 B per cell); a marked point adds its contributions, which the previous step's launch
@@ -118,8 +118,8 @@ __global__ __launch_bounds__(256) void acoustic_tables(AcuArgs A, AcuTabs T) {
 }
 
 struct AcuTiles { int ntz, ntx, nyc, chunk; AcuTabs tab; };
-// Planes per workgroup: as few as keep the workgroups within one round of the chip (three per
-// CU), at most 6 (on large grids, where several rounds run anyway, 5 to 10 measured alike and
+// Planes per workgroup: as few as keep the workgroups within one round of the chip (three on each
+// of 256 CUs), at most 6 (on large grids, where several rounds run anyway, 5 to 10 measured alike and
 // 3 and 16 slower). chunk > 0: by hand (any count: past ny it is the whole axis).
 inline AcuTiles acoustic_tiles(const Geom& g, int chunk) {
     AcuTiles T{};

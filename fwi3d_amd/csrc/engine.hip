@@ -416,7 +416,7 @@ void fused_tables(hipStream_t st, bool vti, const EArgs& A, float* base, FusedTi
 // class: w the iterations that fill its queues, k the cost of an iteration, a middle tile's
 // being 1 (side 1.05, corner 1.7; a y-face workgroup 9: fitted to sweeps). The y chunks are
 // those that give the march classes one time T, for the least estimated step: the work over
-// the slots (two workgroups per CU) and half of T for the ragged end, at least T and a y-face
+// the slots (two workgroups on each of 256 CUs) and half of T for the ragged end, at least T and a y-face
 // workgroup's time where few workgroups leave slots idle. The best and worst elastic steps of
 // sweeps over (middle, side) chunks of 4..63 planes: 200^3 183 and 295 us, 256^3 306 and 423,
 // (ny, nx, nz) = (61, 75, 68) 33 and 181. fchunk / echunk set the middle / side tiles' by
@@ -1036,10 +1036,10 @@ void propagate_elastic(fwi3d_ctx* c, bool vti, bool adj, const float* d_model, c
     };
     // fields of local step k: prev = F[k % 3], curr = F[(k + 1) % 3] (the kernels' rotation)
     auto field = [&](int k) { return F + (long long)(k % 3) * 3 * n; };
-    // one time step: receivers read curr; flux, interior, shell and z slabs write next;
-    // sources add to it (the batch kernels over the one-shot table: a batched shot runs
-    // the same code)
-    // receivers are extracted by workgroups of the shell launch
+    // one time step: receivers read curr; the step's kernels write next; sources add to it (the
+    // batch kernels over the one-shot table: a batched shot runs the same code)
+    // receivers are extracted by the last workgroups of the step's launch (the slab launch of the
+    // several-launch and flux forms)
     const int ext_blk = (!adj && E.npts > 0) ? extract_blocks(E.npts, 3, fused ? FTHREADS : 256) : 0;
     auto step = [&](StepIdx si) {
         timed(c, 4, [&] {

@@ -26,10 +26,12 @@
 // the edge tiles took 185 VGPRs and one workgroup per CU: 144 us of the elastic step at
 // 200^3, now 94 us as a launch of its own.
 //
-// All tiles are one launch. At 200^3 (elastic, MI355X): 183 us per step, against 257 us with
-// the y faces left to a flux pass and slab kernels (82 us alone) and the edge tiles as a
-// launch on a second stream; VTI (nz, nx, ny) = (200, 160, 160) 188 against 282 us, (71, 144,
-// 150) 76 against 150 us; elastic (68, 75, 61) 36 against 92 us. What bounds it: HBM traffic
+// All tiles are one launch. Steps with their injection launch of 5 to 6 us (MI355X, HIP events,
+// the chunks of fused_plan): elastic 200^3 196 us (191 the step's launch alone, by a kernel trace;
+// 187 with the autotuner's chunks), against 253 us, without injection, where the y faces are left to
+// a flux pass and slab kernels (82 us alone) and the edge tiles are a launch on a second stream; 256^3
+// 312 against 437 us; (ny, nx, nz) = (61, 75, 68) 37 against 90 us; VTI (160, 160, 200) 190 against
+// 282 us, (150, 144, 71) 92 (81 with the autotuner's chunks) against 141 us. What bounds it: HBM traffic
 // and vector issue together (middle tiles alone: 5.1 TB/s of measured traffic, the rate of a
 // plain copy, and 55 % of the issue slots).
 //

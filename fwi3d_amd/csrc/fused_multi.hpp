@@ -12,7 +12,7 @@
 // kernels of elastic.hpp. Tiles of 32 z x 16 x points and 512 threads march along y, as in
 // fused.hpp, but with the y neighbours in register queues, four ring planes and one barrier
 // per plane, and the closure rows of all outputs of a site in one row switch (edge tiles: 185
-// VGPRs, one workgroup per CU). 257 us per elastic step at 200^3 (the one-launch step: 183).
+// VGPRs, one workgroup per CU). 253 us per elastic step at 200^3 (the one-launch step: 191).
 #pragma once
 #include "fused.hpp"
 
