@@ -150,7 +150,9 @@ struct InjMap {
     int nv;
 };
 
-// Sum of the injection at point p onto val; scale: the last taper factor, which the values lack.
+// Sum of the injection at point p onto val, in the order of the list; scale: the last taper factor,
+// which the values lack. Four loads are in flight: with one at a time a plane of 4 receivers per
+// point (100^3, adjoint) took 76 us per step, now 39; a launch of its own takes 57.
 __device__ __forceinline__ float inject_at(const InjMap& M, const InjTab& I, unsigned p, int k, float scale, float val) {
     const unsigned bit = p & 31u;
     const GAS unsigned* word = gas((const unsigned*)M.mask) + 2 * (p >> 5);
@@ -159,7 +161,12 @@ __device__ __forceinline__ float inject_at(const InjMap& M, const InjTab& I, uns
     const int j = gas(M.perm)[w.y + __popc(w.x & ((1u << bit) - 1u))];
     const int e1 = gas(I.tbeg)[j + 1];
     const float* V = M.V + (size_t)(k & 1) * M.nv;
-    for (int e = gas(I.tbeg)[j]; e < e1; e++) val = __builtin_fmaf(gas(V)[e], scale, val);
+    int e = gas(I.tbeg)[j];
+    for (; e + 4 <= e1; e += 4) {
+        const float v0 = gas(V)[e], v1 = gas(V)[e + 1], v2 = gas(V)[e + 2], v3 = gas(V)[e + 3];
+        val = __builtin_fmaf(v3, scale, __builtin_fmaf(v2, scale, __builtin_fmaf(v1, scale, __builtin_fmaf(v0, scale, val))));
+    }
+    for (; e < e1; e++) val = __builtin_fmaf(gas(V)[e], scale, val);
     return val;
 }
 

@@ -195,3 +195,66 @@ def test_fused_step_every_point_matches_oracle(eng, shape, case, ychunk):
         last = np.abs(got[:, :, -1] - want[:, :, -1]).max() / np.abs(want[:, :, -1]).max()
         print(f"  fused={fused}: rel L2 vs oracle {rel(got, want):.2e}, worst point of the last sample {last:.2e}")
         assert np.isfinite(got).all() and rel(got, want) <= TRACE_TOL and last <= 10 * TRACE_TOL
+
+
+@pytest.mark.parametrize("npts", [1, 2, 3, 5, 38])
+def test_overlapping_sources_alone_and_in_a_batch(eng, npts):
+    """Sources within two cells of each other, up to some hundred contributions to a point: traces
+    against the oracle, and a batched shot with the same bits."""
+    import torch
+    nt, dt = 80, 0.001
+    model, _, _, rloc, d = small_shot(nt=nt)
+    shape = model.shape[-3:]
+    rng = np.random.default_rng(npts)
+    sloc = (np.array([0.19, 0.17, 0.16]) + rng.uniform(0, 2 * d[0], (npts, 3))).astype(np.float32)
+    src = (W.ricker(25.0, nt, dt)[None, None, :] * rng.uniform(0.5, 1.5, (1, npts, 1))).astype(np.float32)
+    cfg = CASES["free+absorb+taper"]
+    inj, ext = F.Injector(0, sloc, shape, d), F.Injector(0, rloc, shape, d)
+    par = F.make_param(nt, dt, bc=cfg["bc"], taper=cfg["taper"])
+    got = eng.propagate("acoustic", model, src, inj, ext, par, d)
+    want, _ = O.propagate("acoustic", model, src, O.Injector(0, sloc, shape, d, (0, 0, 0)),
+                          O.Injector(0, rloc, shape, d, (0, 0, 0)), O.make_par(nt, 0, dt, bc=cfg["bc"], taper=cfg["taper"]),
+                          d, s="f")
+    print(f"  {npts} sources: rel L2 vs oracle {rel(got, want):.2e}")
+    assert np.abs(want).max() > 0 and rel(got, want) <= TRACE_TOL
+    m, s = torch.from_numpy(np.ascontiguousarray(model)).to("cuda:0"), torch.from_numpy(src).to("cuda:0")
+    r = torch.zeros((1, ext.npts, nt), device="cuda:0")
+    torch.cuda.synchronize()
+    b = F.Batch(eng)
+    b.add("acoustic", m.data_ptr(), s.data_ptr(), r.data_ptr(), inj, ext, par, shape, d)
+    b.run()
+    b.close()
+    assert np.array_equal(r.cpu().numpy(), got)
+
+
+def test_dense_receivers_do_not_slow_the_adjoint_step(eng):
+    """Four receivers per grid point of a plane, injected by an adjoint run (some hundred
+    contributions per point): the one-launch step takes no longer than the interior / shell
+    step with an injection launch."""
+    import torch
+    n, nr, nt, h = 100, 200, 66, 0.01
+    shape, d = (n, n, n), (h, h, h)
+    dev = torch.device("cuda:0")
+    m = torch.stack([torch.full(shape, v, device=dev) for v in (8.0, 0.4)]).contiguous()
+    a = np.linspace(0.05, 0.95, nr) * (n - 1) * h
+    g1, g2 = np.meshgrid(a, a)
+    inj = F.Injector(0, np.stack([g1.ravel(), 0 * g1.ravel() + 0.5 * (n - 1) * h, g2.ravel()], 1).astype(np.float32), shape, d)
+    src = torch.rand((1, nr * nr, nt), device=dev)
+    torch.cuda.synchronize()
+    us = {}
+    try:
+        for fused in (True, False):
+            eng.tune(fused=fused)
+            best = 1e30
+            for _ in range(3):
+                eng.profile(True, steps_only=True)
+                eng.propagate_device("acoustic", m.data_ptr(), src.data_ptr(), 0, inj, None,
+                                     F.make_param(nt, 0.0005, bc=(1, 2, 2, 2, 2, 2)), shape, d, adj=True)
+                ms, k = eng.profile_read(4)  # (replayed windows: the injection included)
+                best = min(best, 1e3 * ms / k)
+            us[fused] = best
+    finally:
+        eng.profile(False)
+        eng.tune(fused=True)
+    print(f"  us per step: one launch {us[True]:.1f}, interior / shell and injection {us[False]:.1f}")
+    assert us[True] <= 1.1 * us[False]
