@@ -322,11 +322,10 @@ typedef struct fwi3d_batch fwi3d_batch;
 int fwi3d_batch_create(fwi3d_ctx *ctx, fwi3d_batch **out);
 int fwi3d_batch_destroy(fwi3d_batch *b);
 /* Device bytes one shot holds while in a batch, at most (for admission by memory footprint);
- * -1 for invalid arguments. That is with the boundary coefficients of the one-launch step: a
- * forward shot with a snapshot store holds none, and a shot for which they cannot be allocated
- * takes the step form that needs none (its results then agree to rounding). A server admits a
- * request by what its own shots hold, without the coefficients where its whole budget has no
- * room for them. */
+ * -1 for invalid arguments. That is with room for the boundary coefficients of the one-launch
+ * step where a shot or its adjoint takes it; a shot for which they cannot be allocated takes the
+ * step form that needs none (its results then agree to rounding). A server admits a request by
+ * what its own shots hold, without the coefficients where its whole budget has no room for them. */
 long long fwi3d_batch_footprint(int physics, int nx, int ny, int nz, const fwi3d_injector *inj,
                                 const fwi3d_injector *ext);
 /* Admit a shot; it starts at the batch's next step. *id identifies it in queries. */

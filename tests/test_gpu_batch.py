@@ -295,29 +295,36 @@ def test_online_tuning_waits_for_a_shot_that_reads_the_chunk():
 
 
 @pytest.mark.parametrize("physics,shape", [("acoustic", (40, 44, 48)), ("vti", (200, 12, 20))])
-def test_store_shots_hold_no_boundary_tables(physics, shape):
-    """A forward shot with a snapshot store does not take the one-launch step: it holds fields,
-    model, fluxes and small tables, not the boundary coefficients (at 384 B per point of a face
-    more than the fluxes on a narrow grid)."""
+def test_shots_hold_the_memory_of_their_step_form(physics, shape):
+    """Without the one-launch step a shot holds fields, model, fluxes and small tables, not the
+    boundary coefficients (at 384 B per point of a face more than the fluxes on a narrow grid);
+    the forward shot of a gradient holds the block that its adjoint takes over."""
     import torch
     dev = torch.device("cuda:0")
     nt = 12
     s = make_shot(physics, shape, nt, 3)
     ny, nx, nz = shape
     cells = ny * nx * ((nz + 63) // 64 * 64)
+    fields = {"acoustic": 3 + 2, "elastic": 9 + 3 + 7, "vti": 9 + 7 + 9}[physics] * cells * 4
+    fp = F.Batch.footprint(physics, shape, s["inj"], s["ext"])
+    assert fp > fields + (1 << 20)
+    held = {}
     eng = F.Engine(0)
     try:
-        b = F.Batch(eng)
         m, src = torch.from_numpy(s["model"]).to(dev), torch.from_numpy(s["src"]).to(dev)
         r = torch.zeros((F.n_comp(F.PHYSICS[physics]), s["ext"].npts, nt), device=dev)
         torch.cuda.synchronize()
-        b.add(physics, m.data_ptr(), src.data_ptr(), r.data_ptr(), s["inj"], s["ext"],
-              F.make_param(nt, DT, sub=3), shape, (H, H, H))
-        held = b.status()[1] - F.Batch.snap_footprint(physics, shape, nt, 3)
-        b.run()
-        b.close()
+        for fused in (False, True):
+            eng.tune(fused=fused)
+            for sub in (0, 3):
+                b = F.Batch(eng)
+                b.add(physics, m.data_ptr(), src.data_ptr(), r.data_ptr(), s["inj"], s["ext"],
+                      F.make_param(nt, DT, sub=sub), shape, (H, H, H))
+                held[fused, sub] = b.status()[1] - (F.Batch.snap_footprint(physics, shape, nt, sub) if sub else 0)
+                b.run()
+                b.close()
     finally:
         eng.close()
-    fields = {"acoustic": 3 + 2, "elastic": 9 + 3 + 7, "vti": 9 + 7 + 9}[physics] * cells * 4
-    assert fields <= held <= fields + (64 << 10)  # injector, taper tables and alignment
-    assert F.Batch.footprint(physics, shape, s["inj"], s["ext"]) > held + (1 << 20)
+    for sub in (0, 3):
+        assert fields <= held[False, sub] <= fields + (64 << 10)  # injector, taper tables and alignment
+        assert held[True, sub] == fp
